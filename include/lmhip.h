@@ -177,6 +177,10 @@ int lmh_solver_order(lmh_context *ctx, int32_t *K, double *s);
 /* A density matrix owned by the library (P plus its two evolution caches,
  * src/evolution.jl:80,188-196).  Contents undefined until uploaded. */
 int lmh_state_create(lmh_context *ctx, lmh_state **st);
+/* Waits for the device.  The state's buffers may stay with the context for
+ * its next states and kets of that size (at most a quarter of the device's
+ * memory over all contexts); they are freed when the context's geometry is
+ * set again, when it is destroyed, and when the library needs the memory. */
 int lmh_state_destroy(lmh_state *st);
 /* Host <-> device copies of P (column-major, leading dimension ld >= N). */
 int lmh_state_upload(lmh_state *st, const double *P, int64_t ld);

@@ -2,6 +2,8 @@
 // (create, destroy, options, profiling, the autotuner, sync) and the
 // context checks every entry point runs.
 
+#include <mutex>
+
 #include "api_internal.h"
 
 using namespace lmhapi;
@@ -23,6 +25,106 @@ int hipfail(hipError_t e, const char *what) {
     return fail(e == hipErrorOutOfMemory ? LMH_ENOMEM : LMH_EDEVICE, "%s: %s", what, hipGetErrorString(e));
 }
 
+namespace {
+
+struct Spare {
+    lmh_context *ctx;
+    int device;
+    void *p;
+    size_t bytes;
+};
+
+// (never destroyed: handles may be released while the process ends)
+std::mutex &spare_mutex() {
+    static std::mutex *m = new std::mutex;
+    return *m;
+}
+std::vector<Spare> &spares() {
+    static std::vector<Spare> *v = new std::vector<Spare>;
+    return *v;
+}
+
+template <class F>
+size_t spare_free_if(F match) {
+    std::lock_guard<std::mutex> lock(spare_mutex());
+    auto &v = spares();
+    size_t freed = 0;
+    for (size_t k = 0; k < v.size();) {
+        if (!match(v[k])) {
+            ++k;
+            continue;
+        }
+        (void)hipFree(v[k].p);          // waits for the device
+        freed += v[k].bytes;
+        v[k] = v.back();
+        v.pop_back();
+    }
+    return freed;
+}
+
+}  // namespace
+
+hipError_t device_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || spare_free_if([dev](const Spare &s) { return s.device == dev; }) == 0)
+        return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
+hipError_t spare_take(lmh_context *ctx, size_t bytes, void **out) {
+    {
+        std::lock_guard<std::mutex> lock(spare_mutex());
+        auto &v = spares();
+        for (size_t k = 0; k < v.size(); ++k)
+            if (v[k].ctx == ctx && v[k].bytes == bytes) {
+                *out = v[k].p;
+                v[k] = v.back();
+                v.pop_back();
+                return hipSuccess;
+            }
+    }
+    return device_malloc(out, bytes);
+}
+
+void spare_give(lmh_context *ctx, void *p, size_t bytes) {
+    if (ctx) {
+        std::lock_guard<std::mutex> lock(spare_mutex());
+        auto &v = spares();
+        size_t mine = 0, held = 0;
+        for (const Spare &s : v) {
+            if (s.ctx == ctx) ++mine;
+            if (s.device == ctx->device) held += s.bytes;
+        }
+        if (mine < kSparesPerContext && held + bytes <= ctx->mem_total / 4) {
+            try {
+                v.push_back({ctx, ctx->device, p, bytes});
+                return;
+            } catch (const std::bad_alloc &) {
+            }
+        }
+    }
+    (void)hipFree(p);
+}
+
+size_t spare_bytes(int device) {
+    std::lock_guard<std::mutex> lock(spare_mutex());
+    size_t held = 0;
+    for (const Spare &s : spares())
+        if (s.device == device) held += s.bytes;
+    return held;
+}
+
+void spare_release(int device) {
+    spare_free_if([device](const Spare &s) { return s.device == device; });
+}
+
+void spare_release_context(lmh_context *ctx) {
+    spare_free_if([ctx](const Spare &s) { return s.ctx == ctx; });
+}
+
 void pool_free(lmh_context *ctx) {
     for (double2 *&p : ctx->pool) dfree(p);
     ctx->pool.clear();
@@ -39,7 +141,7 @@ hipError_t pool_take(lmh_context *ctx, int64_t elems, double2 **out) {
         ctx->pool.pop_back();
         return hipSuccess;
     }
-    return dalloc(out, (size_t)elems);
+    return salloc(ctx, out, (size_t)elems);
 }
 
 hipError_t readback_sync(lmh_context *ctx, const Readback *r, int count) {
@@ -197,6 +299,8 @@ int lmh_create(lmh_context **out, int device) {
     if (!ctx) return fail(LMH_ENOMEM, "host allocation failed");
     ctx->device = device;
     hipError_t e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
+    size_t free_b = 0;
+    if (e == hipSuccess) e = hipMemGetInfo(&free_b, &ctx->mem_total);
     if (e == hipSuccess) e = dalloc(&ctx->d_maxbits, lmh::kMaxTaylor);
     if (e == hipSuccess) e = dalloc(&ctx->d_partmax, (size_t)lmh::taylor_order_scratch());
     if (e == hipSuccess) e = dalloc(&ctx->d_overflow, 1);
@@ -240,6 +344,7 @@ int lmh_destroy(lmh_context *ctx) {
     for (lmh_series *q : std::vector<lmh_series *>(ctx->series.begin(), ctx->series.end())) lmh_series_destroy(q);
     tape_clear(ctx);
     pool_free(ctx);
+    spare_release_context(ctx);
     csc_release(ctx);
     dfree(ctx->adj_partial);
     dfree(ctx->d_tape_fields);

@@ -352,6 +352,7 @@ int lmh_set_geometry(lmh_context *ctx, int64_t nsites, int64_t nbonds, const int
     std::vector<double> onsite_keep = ctx->onsite_host;
     tape_clear(ctx);
     pool_free(ctx);
+    spare_release_context(ctx);
     free_geometry(ctx->h);
     lmh::DevHam &h = ctx->h;
     h.n = n;

@@ -39,11 +39,15 @@ int hipfail(hipError_t e, const char *what);
 
 namespace lmhapi {
 
+// hipMalloc; when the device is full, the spare buffers on it (below) are
+// given back and the allocation is tried once more
+hipError_t device_malloc(void **p, size_t bytes);
+
 template <class T>
 hipError_t dalloc(T **p, size_t count) {
     *p = nullptr;
     if (count == 0) return hipSuccess;
-    return hipMalloc((void **)p, count * sizeof(T));
+    return device_malloc((void **)p, count * sizeof(T));
 }
 
 template <class T>
@@ -69,11 +73,53 @@ hipError_t grow(T *&p, size_t &cap, size_t count) {
 
 }  // namespace lmhapi
 
+struct lmh_context;
+
+namespace lmhapi {
+
+// Buffers of destroyed states and kets, kept for the context's next state of
+// the same size: an evolution that starts from a kept P0 would otherwise pay
+// three N x N hipMalloc and hipFree (1.0 ms at N = 10^4, and at N = 28800,
+// once the driver has to clear the memory it hands out, 0.8 s).  Reuse stays
+// within one context, hence in its stream's order.  Bounded: kSparesPerContext
+// buffers of a context, a quarter of the device's memory over all contexts;
+// given back when the context's geometry changes or it is destroyed, when an
+// allocation fails, and before library calls that allocate by themselves.
+constexpr size_t kSparesPerContext = 16;
+hipError_t spare_take(lmh_context *ctx, size_t bytes, void **out);
+void spare_give(lmh_context *ctx, void *p, size_t bytes);
+size_t spare_bytes(int device);
+void spare_release(int device);
+void spare_release_context(lmh_context *ctx);
+
+template <class T>
+hipError_t salloc(lmh_context *ctx, T **p, size_t count) {
+    *p = nullptr;
+    return count ? spare_take(ctx, count * sizeof(T), (void **)p) : hipSuccess;
+}
+template <class T>
+void sfree(lmh_context *ctx, T *&p, size_t count) {
+    if (p) spare_give(ctx, p, count * sizeof(T));
+    p = nullptr;
+}
+template <class T>
+hipError_t grow_spare(lmh_context *ctx, T *&p, size_t &cap, size_t count) {
+    if (count <= cap) return hipSuccess;
+    sfree(ctx, p, cap);
+    cap = 0;
+    hipError_t e = salloc(ctx, &p, count);
+    if (e == hipSuccess) cap = count;
+    return e;
+}
+
+}  // namespace lmhapi
+
 struct lmh_state;
 
 struct lmh_context {
     int device = 0;
     hipStream_t stream = nullptr;
+    size_t mem_total = 0;                 // the device's memory
     lmh_progress_fn progress = nullptr;   // lmh_set_progress
     void *progress_user = nullptr;
     lmh::DevHam h;

@@ -22,7 +22,7 @@ int lmh_kets_create(lmh_context *ctx, int64_t m, lmh_kets **out) {
     k->m = m;
     k->ld = ((ctx->h.n + 7) / 8) * 8;
     for (int b = 0; b < 3; ++b) {
-        hipError_t e = dalloc(&k->buf[b], (size_t)k->ld * m);
+        hipError_t e = salloc(ctx, &k->buf[b], (size_t)k->ld * m);
         if (e != hipSuccess) {
             for (int q = 0; q < 3; ++q) dfree(k->buf[q]);
             delete k;
@@ -38,15 +38,15 @@ int lmh_kets_destroy(lmh_kets *k) {
     if (!k) return LMH_OK;
     if (k->ctx) {
         (void)hipSetDevice(k->ctx->device);
-        (void)hipStreamSynchronize(k->ctx->stream);
+        (void)hipDeviceSynchronize();
         k->ctx->kets.erase(k);
     }
-    for (int q = 0; q < 3; ++q) dfree(k->buf[q]);
+    for (int q = 0; q < 3; ++q) sfree(k->ctx, k->buf[q], (size_t)k->ld * k->m);
     krylov_graphs_free(k);
-    dfree(k->basis);
-    dfree(k->lz);
-    dfree(k->coef);
-    dfree(k->len);
+    sfree(k->ctx, k->basis, k->basis_cap);
+    sfree(k->ctx, k->lz, k->lz_cap);
+    sfree(k->ctx, k->coef, k->coef_cap);
+    sfree(k->ctx, k->len, k->len_cap);
     if (k->h_pin) (void)hipHostFree(k->h_pin);
     delete k;
     return LMH_OK;
@@ -161,10 +161,10 @@ int lmh_krylov_step(lmh_context *ctx, lmh_kets *k, double dt, int krylovdim, dou
         (size_t)m * kd > k->coef_cap || (size_t)m > k->len_cap || pin_need > k->h_pin_cap)
         HIP_TRY(hipStreamSynchronize(st), "hipStreamSynchronize");
     // basis v_0 .. v_{kd-1}, then two scratch blocks for the unnormalised w
-    HIP_TRY(grow(k->basis, k->basis_cap, (size_t)(kd + 2) * vstride), "Krylov basis allocation");
-    HIP_TRY(grow(k->lz, k->lz_cap, nalpha + nbeta + 3 * npart), "Krylov work allocation");
-    HIP_TRY(grow(k->coef, k->coef_cap, (size_t)m * kd), "Krylov work allocation");
-    HIP_TRY(grow(k->len, k->len_cap, (size_t)m), "Krylov work allocation");
+    HIP_TRY(grow_spare(ctx, k->basis, k->basis_cap, (size_t)(kd + 2) * vstride), "Krylov basis allocation");
+    HIP_TRY(grow_spare(ctx, k->lz, k->lz_cap, nalpha + nbeta + 3 * npart), "Krylov work allocation");
+    HIP_TRY(grow_spare(ctx, k->coef, k->coef_cap, (size_t)m * kd), "Krylov work allocation");
+    HIP_TRY(grow_spare(ctx, k->len, k->len_cap, (size_t)m), "Krylov work allocation");
     if (pin_need > k->h_pin_cap) {
         if (k->h_pin) (void)hipHostFree(k->h_pin);
         k->h_pin = nullptr;

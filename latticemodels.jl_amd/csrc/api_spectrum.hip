@@ -24,6 +24,7 @@ int eigensolve(lmh_context *ctx, double2 *A, int64_t lda, std::vector<double> &E
         HIP_TRY(lmh::launch_build_h(h, ctx->stream), "build_h launch");
         ctx->built_version = ctx->param_version;
     }
+    spare_release(ctx->device);             // rocSOLVER allocates its own work space
     const int64_t n = h.n;
     double *dE = nullptr, *dwork = nullptr, *R = nullptr;
     int *dinfo = nullptr;

@@ -18,7 +18,7 @@ int lmh_state_create(lmh_context *ctx, lmh_state **out) {
     st->n = ctx->h.n;
     st->ld = ((ctx->h.n + 7) / 8) * 8;
     for (int b = 0; b < 3; ++b) {
-        hipError_t e = dalloc(&st->buf[b], (size_t)st->ld * st->n);
+        hipError_t e = salloc(ctx, &st->buf[b], (size_t)st->ld * st->n);
         if (e != hipSuccess) {
             for (int q = 0; q < 3; ++q) dfree(st->buf[q]);
             delete st;
@@ -35,14 +35,17 @@ int lmh_state_destroy(lmh_state *st) {
     if (st->ctx) {
         (void)hipSetDevice(st->ctx->device);
         (void)ctx_resolve(st->ctx);          // the journal may name this state
-        (void)hipStreamSynchronize(st->ctx->stream);
+        // the whole device, as hipFree waits: the caller's own streams may
+        // still read the pointer of lmh_state_device_ptr, and the buffers are
+        // used again without a hipFree in between
+        (void)hipDeviceSynchronize();
         st->ctx->states.erase(st);
         if (st->ctx->tape.st == st) tape_clear(st->ctx);
     }
-    for (int q = 0; q < 3; ++q) dfree(st->buf[q]);
-    dfree(st->pend_stval);
-    dfree(st->pend_sdiag);
-    dfree(st->pend_coef);
+    for (int q = 0; q < 3; ++q) sfree(st->ctx, st->buf[q], (size_t)st->ld * st->n);
+    sfree(st->ctx, st->pend_stval, (size_t)st->pend_cap_stval);
+    sfree(st->ctx, st->pend_sdiag, (size_t)st->pend_cap_sdiag);
+    sfree(st->ctx, st->pend_coef, 1);
     delete st;
     return LMH_OK;
 }
@@ -184,6 +187,7 @@ int lmh_state_idempotency(lmh_state *st, double *max_err) {
     HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     double2 *W = nullptr;
     HIP_TRY(pool_take(ctx, st->ld * st->n, &W), "idempotency scratch");
+    spare_release(ctx->device);             // rocBLAS allocates its own work space
     constexpr int kBlocks = 1024;
     hipError_t e = grow(ctx->xfer, ctx->xfer_cap, (size_t)8 * kBlocks);
     int s = e == hipSuccess ? lmh::idempotency(ctx->stream, st->buf[st->cur], st->n, st->ld, W,
@@ -360,15 +364,15 @@ int step_impl(lmh_context *ctx, lmh_state *st) {
                 HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
                 dfree(st->pend_stval);
                 st->pend_cap_stval = 0;
-                HIP_TRY(dalloc(&st->pend_stval, (size_t)nsv), "deferred pass allocation");
+                HIP_TRY(salloc(ctx, &st->pend_stval, (size_t)nsv), "deferred pass allocation");
                 st->pend_cap_stval = nsv;
             }
-            if (!st->pend_coef) HIP_TRY(dalloc(&st->pend_coef, 1), "deferred pass allocation");
+            if (!st->pend_coef) HIP_TRY(salloc(ctx, &st->pend_coef, 1), "deferred pass allocation");
             if (st->pend_cap_sdiag < nsd) {
                 HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
                 dfree(st->pend_sdiag);
                 st->pend_cap_sdiag = 0;
-                HIP_TRY(dalloc(&st->pend_sdiag, (size_t)nsd), "deferred pass allocation");
+                HIP_TRY(salloc(ctx, &st->pend_sdiag, (size_t)nsd), "deferred pass allocation");
                 st->pend_cap_sdiag = nsd;
             }
             {

@@ -31,7 +31,7 @@ hipError_t checkpoint_alloc(lmh_context *ctx, int64_t elems, double2 **out, bool
         if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) {
             const size_t pooled = elems == ctx->pool_elems ? ctx->pool.size() * bytes : 0;
             const size_t reserve = bytes * (size_t)(7 + std::max(ctx->K - 1, 0)) + ((size_t)8 << 30);
-            want_host = free_b + pooled < bytes + reserve;
+            want_host = free_b + spare_bytes(ctx->device) + pooled < bytes + reserve;
         }
     }
     if (want_host) {
@@ -257,7 +257,9 @@ int lmh_tape_backward(lmh_context *ctx, lmh_state *lam, double *grad_field, doub
             double2 *p = nullptr;
             if (ctx->pool.empty() || ctx->pool_elems != ld * n) {
                 size_t free_b = 0, total_b = 0;
-                if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < bytes + ((size_t)4 << 30)) break;
+                if (hipMemGetInfo(&free_b, &total_b) != hipSuccess ||
+                    free_b + spare_bytes(ctx->device) < bytes + ((size_t)4 << 30))
+                    break;
             }
             if (pool_take(ctx, ld * n, &p) != hipSuccess) break;
             iters.push_back(p);

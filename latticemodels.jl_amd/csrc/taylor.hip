@@ -611,7 +611,7 @@ hipError_t launch_grid_t(const DevHam &h, double dt, double nztol, const TaylorR
     constexpr int D = 2 * R * R + 2 * R + 1;
     const size_t lds = (size_t)kGridWaves * 2 * D * sizeof(double2);
     static std::atomic<uint64_t> done{0};
-    hipError_t e = once_per_device(done, [lds] {
+    hipError_t e = once_per_device(done, [] {
         return hipFuncSetAttribute((const void *)taylor_grid_kernel<R, kGridWaves>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
