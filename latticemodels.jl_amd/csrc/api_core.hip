@@ -435,6 +435,7 @@ int lmh_set_option(lmh_context *ctx, int key, int64_t value) {
         case LMH_OPT_RIGHT_PASS:
             if (value < 1 || value > 5) return fail(LMH_EINVAL, "right-pass variant must be 1 .. 5");
             ctx->right_variant = (int)value;
+            ctx->right_set = true;
             return LMH_OK;
         case LMH_OPT_LEFT_PASS:
             if (value < 0 || value > 3) return fail(LMH_EINVAL, "left-pass variant must be 0 .. 3");
@@ -563,12 +564,12 @@ int lmh_autotune(lmh_context *ctx, lmh_state *st, int32_t reps, double *best_ms)
     for (int lc : {16, 32, 64}) {
         // both sides as left passes (banded and gather kernels when the band fits)
         for (int rv : {1, 5}) {
-            cands.push_back({LMH_STEP_PER_PASS, rv, lc, 16, -1, 0});
+            cands.push_back({LMH_STEP_PER_PASS, rv, lc, 16, -1, band ? 2 : 0});
             if (band) cands.push_back({LMH_STEP_PER_PASS, rv, lc, 16, -1, 1});
             if (lmh::left_band2_fits(ctx->h)) cands.push_back({LMH_STEP_PER_PASS, rv, lc, 16, -1, 3});
         }
         for (int rv : {3, 4})
-            for (int rcol : {4, 8, 16, 32}) cands.push_back({LMH_STEP_PER_PASS, rv, lc, rcol, -1, 0});
+            for (int rcol : {4, 8, 16, 32}) cands.push_back({LMH_STEP_PER_PASS, rv, lc, rcol, -1, band ? 2 : 0});
     }
     if (lmh::fused_supported(ctx->h)) {
         for (int v = 0; v < lmh::fused_variant_count(); ++v) {
@@ -585,9 +586,11 @@ int lmh_autotune(lmh_context *ctx, lmh_state *st, int32_t reps, double *best_ms)
     }
     const Cfg saved = {ctx->step_mode, ctx->right_variant, ctx->left_cols, ctx->right_cols, ctx->fused_variant,
                        ctx->left_variant};
+    const bool right_was_set = ctx->right_set;
     auto apply = [&](const Cfg &cf) {
         ctx->step_mode = cf.mode;
         ctx->right_variant = cf.rv;
+        ctx->right_set = right_was_set || cf.mode == LMH_STEP_PER_PASS;
         ctx->left_cols = cf.lc;
         ctx->right_cols = cf.rc_;
         ctx->fused_variant = cf.fv;
@@ -624,6 +627,7 @@ int lmh_autotune(lmh_context *ctx, lmh_state *st, int32_t reps, double *best_ms)
     ctx->profiling = prof;
     if (rc || he != hipSuccess) {
         apply(saved);
+        ctx->right_set = right_was_set;
         return rc ? rc : hipfail(he, "autotune timing");
     }
     apply(bestc);

@@ -163,6 +163,7 @@ struct lmh_context {
     std::vector<hipEvent_t> event_pool;
     int step_mode = LMH_STEP_AUTO;
     int right_variant = 3;
+    bool right_set = false;           // LMH_OPT_RIGHT_PASS set (or autotuned), else by step_right
     int left_variant = 0;             // LMH_OPT_LEFT_PASS
     // eigensystem of lmh_diagonalize (eigenvectors N x ld on the device)
     double2 *eigvec = nullptr;
@@ -395,6 +396,8 @@ int check_entries(const lmh_state *st, int64_t count, const int64_t *rows, const
 int step_impl(lmh_context *ctx, lmh_state *st);
 bool step_may_stay(const lmh_context *ctx, const lmh_state *st);
 int step_async(lmh_context *ctx, lmh_state *st);
+int step_left(const lmh_context *ctx);
+int step_right(const lmh_context *ctx);
 int ensure_built(lmh_context *ctx);
 int upload_mask(const uint8_t *mask, int64_t n, uint8_t **dev);
 int eigensolve(lmh_context *ctx, double2 *A, int64_t lda, std::vector<double> &E);

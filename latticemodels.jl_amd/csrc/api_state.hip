@@ -214,6 +214,19 @@ namespace lmhapi {
 
 int step_impl(lmh_context *ctx, lmh_state *st);
 
+// The per-term schedule where the caller has set none.  The banded left pass
+// streams whole columns (7.0 ms per term at N = 28800, 9 neighbours per site;
+// two terms per launch 11.7 ms) while the right pass sweeps neighbour
+// columns through the caches (18.3 ms per term), so both sides run as left
+// passes with a tiled conjugate transpose (5.0 ms) between them wherever the
+// band fits: a step takes 75 instead of 152 ms at K = 6.
+int step_left(const lmh_context *ctx) {
+    return ctx->left_variant == 0 && lmh::left_band2_fits(ctx->h) ? 3 : ctx->left_variant;
+}
+int step_right(const lmh_context *ctx) {
+    return !ctx->right_set && lmh::left_band_fits(ctx->h) && ctx->left_variant != 1 ? 5 : ctx->right_variant;
+}
+
 // a strip step whose polynomial is still on the device (ctx->order_async):
 // the state's own deferred-pass buffers are in place (allocated by an
 // earlier step) and the step runs on the strip path
@@ -422,15 +435,20 @@ int step_impl(lmh_context *ctx, lmh_state *st) {
         if (!keep_form) st->conj ^= 1;
         return LMH_OK;
     }
-    // the per-term passes work on P itself
-    rc = state_normalize(st);
-    if (rc) return rc;
     // right_variant 1: both sides as left passes, each side's last term
     // written conjugate-transposed: (U (U P)')' = U P U' for any P;
     // right_variant 5: the same with each side's result transposed by the
     // tiled transpose kernel instead (coalesced writes)
-    const bool tr = ctx->right_variant == 1 || ctx->right_variant == 5;
-    const bool tr_kernel = ctx->right_variant == 5;
+    const int lv = step_left(ctx), rv = step_right(ctx);
+    const bool tr = rv == 1 || rv == 5;
+    const bool tr_kernel = rv == 5;
+    // with the tiled transposes the second one is left out, as in the fused
+    // steps: from the stored S (P, or P^H when st->conj) U (U S)^H =
+    // (U S U^H)^H, so the state changes form; the other schedules and a state
+    // recorded by a tape (checkpoints are copies of the buffer) work on P
+    const bool flip = tr_kernel && !(ctx->tape.active && ctx->tape.st == st);
+    rc = flip ? state_settle(st) : state_normalize(st);
+    if (rc) return rc;
     int x = st->cur;
     for (int side = 0; side < 2; ++side) {
         for (int r = 0; r < reps; ++r) {
@@ -446,7 +464,7 @@ int step_impl(lmh_context *ctx, lmh_state *st) {
                 const bool tout = tr && !tr_kernel && r == reps - 1 && k == 1;
                 // left variant 3: terms k and k-1 in one launch (not the
                 // conjugate-transposed last term)
-                const bool pair = left && ctx->left_variant == 3 && k >= 2 && !(tr && !tr_kernel && r == reps - 1 && k == 2);
+                const bool pair = left && lv == 3 && k >= 2 && !(tr && !tr_kernel && r == reps - 1 && k == 2);
                 ProfScope ps(ctx, left ? LMH_KERNEL_HORNER_LEFT : LMH_KERNEL_HORNER_RIGHT);
                 hipError_t e;
                 if (pair)
@@ -454,18 +472,18 @@ int step_impl(lmh_context *ctx, lmh_state *st) {
                                                  ctx->dt / (ctx->s * (k - 1)), k == K, ctx->left_cols, ctx->stream);
                 else if (left)
                     e = lmh::launch_horner_left(h, st->buf[x], st->buf[in], st->buf[out], st->ld, st->n, c, k == K,
-                                                ctx->left_cols, ctx->stream, ctx->left_variant == 3 ? 2 : ctx->left_variant,
+                                                ctx->left_cols, ctx->stream, lv == 3 ? 2 : lv,
                                                 tout);
                 else
                     e = lmh::launch_horner_right(h, st->buf[x], st->buf[in], st->buf[out], st->ld, st->n, c, k == K,
-                                                 ctx->right_variant, ctx->right_cols, ctx->stream);
+                                                 rv, ctx->right_cols, ctx->stream);
                 if (e != hipSuccess) return hipfail(e, "horner launch");
                 in = out;
                 k -= pair ? 2 : 1;
             }
             x = in;
         }
-        if (tr_kernel) {
+        if (tr_kernel && !(flip && side == 1)) {
             const int dst = (x + 1) % 3;          // both other buffers are free after the side
             ProfScope ps(ctx, LMH_KERNEL_TRANSPOSE);
             HIP_TRY(lmh::launch_conj_transpose(st->buf[x], st->buf[dst], st->n, st->ld, ctx->stream),
@@ -474,6 +492,7 @@ int step_impl(lmh_context *ctx, lmh_state *st) {
         }
     }
     st->cur = x;
+    if (flip) st->conj ^= 1;
     return LMH_OK;
 }
 

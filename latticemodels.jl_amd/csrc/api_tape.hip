@@ -213,7 +213,7 @@ int lmh_tape_backward(lmh_context *ctx, lmh_state *lam, double *grad_field, doub
     // per-term helpers (any N): y = p(-i a H) x from the left, the result in `out`
     // (with left variant 3, terms k and k-1 in one launch)
     auto left_poly = [&](const lmh::DevHam &hh, const double2 *X, double2 *out, double2 *tmp, double a, int K) {
-        const bool pairs = ctx->left_variant == 3 && lmh::left_band2_fits(hh);
+        const bool pairs = step_left(ctx) == 3 && lmh::left_band2_fits(hh);
         const int nl = pairs ? K / 2 + K % 2 : K;           // launches; the last one writes `out`
         double2 *b[2] = {(nl % 2) ? out : tmp, (nl % 2) ? tmp : out};
         const double2 *yin = X;
@@ -359,7 +359,7 @@ int lmh_tape_backward(lmh_context *ctx, lmh_state *lam, double *grad_field, doub
                 e = cp_host ? hipMemcpyAsync(Pa, ckpt, sizeof(double2) * ld * n, hipMemcpyHostToDevice, st)
                             : lmh::launch_copy(ckpt, Pa, ld * n, st);
             if (e == hipSuccess && !cp) {
-                if (ctx->right_variant == 1 || ctx->right_variant == 5) {
+                if (step_right(ctx) == 1 || step_right(ctx) == 5) {
                     e = lmh::launch_conj_transpose(XA, G1, n, ld, st);
                     if (e == hipSuccess) e = left_poly(hk, G1, Pa, T2, -r.dt, r.K);
                 } else {
