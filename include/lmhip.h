@@ -491,13 +491,14 @@ int lmh_set_step_mode(lmh_context *ctx, int mode);
                                     hoppings are all real goes to the real solvers first */
 #define LMH_OPT_FUSED_VARIANT 7  /* fused column pass shape (threads, sites/thread, columns,
                                     H in registers, x in registers, site H layout): -1 = by
-                                    N, else a variant index (0..32).  Variant 32 is the strip
+                                    N, else a variant index (0..53).  Variant 32 is the strip
                                     kernel for grid-stencil H (square lattices): a thread
                                     owns a run of consecutive sites with its bond values in
                                     registers.  It runs (and is the default) whenever the
                                     geometry is a grid and the last H build gave every
                                     strip uniform bonds (Landau gauge, no field); else the
-                                    by-size default runs */
+                                    by-size default runs.  33..53: the column kernel (H's
+                                    rows in registers or loaded a site ahead) */
 #define LMH_OPT_ADJOINT_MODE 8   /* lmh_tape_backward: 0 = fused when K N <= 10240 (else
                                     per-term), 1 = fused only, 2 = per-term passes (the
                                     K-1 Horner iterates of a side kept in HBM when it has

@@ -158,6 +158,8 @@ void free_geometry(lmh::DevHam &h) {
     dfree(h.cbond);
     dfree(h.col);
     dfree(h.col4);
+    dfree(h.cpk);
+    dfree(h.cpk2);
     dfree(h.val);
     dfree(h.diag);
     dfree(h.rec);
@@ -375,6 +377,24 @@ int lmh_set_geometry(lmh_context *ctx, int64_t nsites, int64_t nbonds, const int
         for (int64_t i = 0; i < n; ++i) col4[((q / 4) * n + i) * 4 + q % 4] = col[q * n + i];
     if (e == hipSuccess) e = dalloc(&h.col, nslots);
     if (e == hipSuccess) e = dalloc(&h.col4, col4.size());
+    // the same columns in 16 bits each (empty slots: the site itself)
+    const bool packed = zmax > 0 && zmax <= 12 && n < 65536;
+    std::vector<uint16_t> c16a, c16b;
+    if (packed) {
+        c16a.resize(8 * n);
+        c16b.resize(4 * n);
+        for (int64_t i = 0; i < n; ++i)
+            for (int q = 0; q < 12; ++q) {
+                const int32_t c = q < zmax ? col[q * n + i] : -1;
+                const uint16_t v = (uint16_t)(c < 0 ? i : c);
+                if (q < 8)
+                    c16a[8 * i + q] = v;
+                else
+                    c16b[4 * i + q - 8] = v;
+            }
+        if (e == hipSuccess) e = dalloc(&h.cpk, n);
+        if (e == hipSuccess) e = dalloc(&h.cpk2, n);
+    }
     // val padded to whole 4-slot chunks of col4; the padding stays zero
     if (e == hipSuccess) e = dalloc(&h.val, zq * 4 * n);
     if (e == hipSuccess) e = hipMemset(h.val, 0, sizeof(double2) * zq * 4 * n);
@@ -399,6 +419,10 @@ int lmh_set_geometry(lmh_context *ctx, int64_t nsites, int64_t nbonds, const int
     up(h.cbond, cbond.data(), 8 * cbond.size());
     up(h.col, col.data(), 4 * nslots);
     up(h.col4, col4.data(), 4 * col4.size());
+    if (packed) {
+        up(h.cpk, c16a.data(), 16 * n);
+        up(h.cpk2, c16b.data(), 8 * n);
+    }
     if (e == hipSuccess) e = lmh::prepare_passes(nullptr);
     // grid-stencil pattern: the strip kernel's geometry and direction slots
     if (e == hipSuccess && n <= 10240) {

@@ -358,7 +358,7 @@ int step_impl(lmh_context *ctx, lmh_state *st) {
         const bool keep_form = ctx->tape.active && ctx->tape.st == st;
         const double dts = ctx->dt / ctx->s;
         const int v = ctx->fused_variant;
-        ctx->fused_launched = lmh::fused_resolved_variant(h, v);
+        ctx->fused_launched = lmh::fused_resolved_variant(h, v, reps);
         const bool defer = mode == LMH_STEP_FUSED_T && ctx->defer && !keep_form &&
                            ctx->fused_launched == lmh::fused_strip_variant();
         if (!defer) {

@@ -445,7 +445,10 @@ hipError_t dispatch(int v, const DevHam &h, const double2 *X, double2 *Y, double
 
 bool fused_supported(const DevHam &h) { return h.n > 0 && h.n <= kFusedMaxN; }
 
-int fused_variant_count() { return kNumVariants + 1; }
+// the column kernel's variants (column.hip) follow the strip kernel's
+constexpr int kColumnVariant0 = kStripVariant + 1;
+
+int fused_variant_count() { return kColumnVariant0 + column_variant_count(); }
 
 int fused_strip_variant() { return kStripVariant; }
 
@@ -453,6 +456,7 @@ bool fused_variant_valid(int v, int64_t n, int zmax) {
     // the strip variant runs where the last H build allows it, else the
     // by-size default: valid wherever a fused pass is
     if (v == kStripVariant) return n > 0 && n <= kFusedMaxN;
+    if (v >= kColumnVariant0) return column_variant_valid(v - kColumnVariant0, n, zmax);
     if (v < 0 || v >= kNumVariants) return false;
     const Variant &w = kVariants[v];
     const int64_t extra = w.zq == 2 ? 4 * kDictMaxOffsets : 0;
@@ -485,11 +489,17 @@ bool fused_dict_fits(int v, int64_t n, int ndict) {
 
 int fused_variant_columns(int v) { return v == kStripVariant ? 1 : kVariants[v].c; }
 
-// Default variant by size, from timing every variant on square lattices
-// (N = 1024 .. 10^4, K = 8): x held in registers wins at every size; H rows in
+// The kernel above by size (batches, and what the column kernel does not
+// take), from timing every variant on square lattices (N = 1024 .. 10^4,
+// K = 8): x held in registers wins at every size; H rows in
 // registers for N <= 1024; above that, for zmax <= 4, the packed site record
 // (diagonal + 16-bit columns, one 16-byte load) beats separate loads by 5-10%.
 int fused_default_variant(int64_t n, int zmax) {
+    const int c = column_default_variant(n, zmax);
+    return c >= 0 ? kColumnVariant0 + c : fused_general_variant(n, zmax);
+}
+
+int fused_general_variant(int64_t n, int zmax) {
     const bool packed = zmax <= 4;
     if (n <= 1024) return packed ? 16 : 19;
     if (n <= 2048) return packed ? 24 : 17;
@@ -499,11 +509,12 @@ int fused_default_variant(int64_t n, int zmax) {
 }
 
 // Default variant of a batch size class.
-int fused_batch_variant(int64_t n, int zmax) { return fused_default_variant(n, zmax); }
+int fused_batch_variant(int64_t n, int zmax) { return fused_general_variant(n, zmax); }
 
-int fused_resolved_variant(const DevHam &h, int variant) {
+int fused_resolved_variant(const DevHam &h, int variant, int reps) {
     if ((variant < 0 || variant == kStripVariant) && h.strip_ok && h.sg.s > 0) return kStripVariant;
     int v = variant < 0 || variant == kStripVariant ? fused_default_variant(h.n, h.zmax) : variant;
+    if (v >= kColumnVariant0 && !column_variant_runs(v - kColumnVariant0, h, reps)) v = fused_general_variant(h.n, h.zmax);
     if (variant < 0 && fused_default_dict(v) >= 0) v = fused_default_dict(v);
     if (fused_variant_is_dict(v) && !(h.ndict > 0 && h.dict_ok && fused_dict_fits(v, h.n, h.ndict)))
         v = fused_variant_fallback(v);
@@ -517,14 +528,12 @@ hipError_t launch_fused_left(const DevHam &h, const double2 *X, double2 *Y, doub
     // the strip kernel by default wherever the last H build allows it
     if ((variant < 0 || variant == kStripVariant) && h.strip_ok && h.sg.s > 0)
         return launch_strip(h, X, Y, ld, ncols, dt_over_s, K, reps, transposed_out, st);
-    if (variant == kStripVariant) variant = -1;
-    if (reps > 1 && !scratch) return hipErrorInvalidValue;
-    int v = variant < 0 ? fused_default_variant(h.n, h.zmax) : variant;
-    if (variant < 0 && fused_default_dict(v) >= 0) v = fused_default_dict(v);
-    // the class table only when the last H build matched it and it fits
-    if (fused_variant_is_dict(v) && !(h.ndict > 0 && h.dict_ok && fused_dict_fits(v, h.n, h.ndict)))
-        v = fused_variant_fallback(v);
+    // (a class table only when the last H build matched it and it fits)
+    const int v = fused_resolved_variant(h, variant, reps);
+    if (v < kColumnVariant0 && reps > 1 && !scratch) return hipErrorInvalidValue;
     if (!fused_variant_valid(v, h.n, h.zmax)) return hipErrorInvalidValue;
+    if (v >= kColumnVariant0)
+        return launch_column(v - kColumnVariant0, h, X, Y, ld, ncols, dt_over_s, K, reps, transposed_out, st);
     return transposed_out ? dispatch<true>(v, h, X, Y, scratch, ld, ncols, dt_over_s, K, reps, st)
                           : dispatch<false>(v, h, X, Y, scratch, ld, ncols, dt_over_s, K, reps, st);
 }

@@ -70,6 +70,8 @@ struct DevHam {
     // Hamiltonian (device)
     int32_t *col = nullptr;     // [zmax*n]
     int32_t *col4 = nullptr;    // [ceil(zmax/4)][n][4]: a site's columns four to a 16-byte record
+    uint4 *cpk = nullptr;       // [n] a site's columns in 16 bits each, slots 0..7 (empty: the site); zmax <= 12, n < 65536
+    uint2 *cpk2 = nullptr;      // [n] slots 8..11
     double2 *val = nullptr;     // [zmax*n] (allocated to whole chunks of col4, padding zero)
     double *diag = nullptr;     // [n]
     double2 *rec = nullptr;     // [n] {diag, four 16-bit columns (empty: 0)}; zmax <= 4, n < 65536 only
@@ -348,6 +350,7 @@ int fused_variant_fallback(int v);
 bool fused_dict_fits(int v, int64_t n, int ndict);
 int fused_variant_columns(int v);
 int fused_default_variant(int64_t n, int zmax);
+int fused_general_variant(int64_t n, int zmax);
 int fused_batch_variant(int64_t n, int zmax);
 hipError_t prepare_fused(int variant);
 // maxdict: the largest class table among the items (value-class variants)
@@ -367,7 +370,16 @@ hipError_t launch_conj_transpose(const double2 *A, double2 *B, int64_t n, int64_
 // the variant number of the strip kernel, and the variant a fused launch with
 // `variant` (-1: default) runs for the current H
 int fused_strip_variant();
-int fused_resolved_variant(const DevHam &h, int variant);
+int fused_resolved_variant(const DevHam &h, int variant, int reps = 1);
+
+// kernels/launchers (column.hip): fused column pass with H's rows in registers
+// or loaded a site ahead; variants (threads, sites per thread, columns, slots)
+int column_variant_count();
+bool column_variant_valid(int v, int64_t n, int zmax);
+bool column_variant_runs(int v, const DevHam &h, int reps);
+int column_default_variant(int64_t n, int zmax);    // -1: the general kernel
+hipError_t launch_column(int v, const DevHam &h, const double2 *X, double2 *Y, int64_t ld, int64_t ncols,
+                         double dt_over_s, int K, int reps, bool tout, hipStream_t st);
 
 // kernels/launchers (adjoint.hip): one side of a reverse step, see adjoint.hip
 struct AdjointSide {
