@@ -161,6 +161,7 @@ void free_geometry(lmh::DevHam &h) {
     dfree(h.cpk);
     dfree(h.cpk2);
     dfree(h.val);
+    dfree(h.hpart);
     dfree(h.diag);
     dfree(h.rec);
     dfree(h.onsite);
@@ -399,6 +400,7 @@ int lmh_set_geometry(lmh_context *ctx, int64_t nsites, int64_t nbonds, const int
     if (e == hipSuccess) e = dalloc(&h.val, zq * 4 * n);
     if (e == hipSuccess) e = hipMemset(h.val, 0, sizeof(double2) * zq * 4 * n);
     if (e == hipSuccess) e = dalloc(&h.diag, n);
+    if (e == hipSuccess) e = dalloc(&h.hpart, 2 * lmh::build_h_parts(n));
     if (e == hipSuccess && zmax <= 4 && n < 65536) e = dalloc(&h.rec, n);
     if (e != hipSuccess) {
         free_geometry(ctx->h);

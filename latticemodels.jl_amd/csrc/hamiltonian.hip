@@ -48,9 +48,28 @@ __device__ __forceinline__ double2 slot_value(const DevHam &h, int64_t q, const 
     return acc;
 }
 
-__global__ void __launch_bounds__(256) build_h_kernel(DevHam h) {
-    __shared__ double red_mx[256], red_rs[256];
-    const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+constexpr int kBuildLdsSlots = 64;
+
+// H's rows, 64 to a workgroup: lane = row, thread row y = its slots y, y +
+// blockDim.y, ... -- a slot's value is a chain of dependent loads and an acos
+// or sincos, so the slots of a row run side by side (one thread per row, slot
+// after slot, took 9-27 us for N = 100 .. 3200).  The row maxima and absolute
+// sums go to one partial per workgroup (no atomics, nothing to clear
+// beforehand), reduced by h_check_kernel; workgroup 0 clears its flags.
+__global__ void __launch_bounds__(1024) build_h_kernel(DevHam h) {
+    extern __shared__ double mag[];                 // [zmax][64] |H_ij|, for zmax <= kBuildLdsSlots
+    const int lane = threadIdx.x;
+    const int64_t r = blockIdx.x * (int64_t)64 + lane;
+    if (blockIdx.x == 0 && lane < 2 && threadIdx.y == 0) h.red[2 + lane] = 0ull;
+    if (r < h.n)
+        for (int s = threadIdx.y; s < h.zmax; s += blockDim.y) {
+            const int64_t q = (int64_t)s * h.n + r;
+            const double2 acc = slot_value(h, q, h.field, h.nfield);
+            h.val[q] = acc;
+            if (h.zmax <= kBuildLdsSlots) mag[s * 64 + lane] = habs(acc);
+        }
+    __syncthreads();
+    if (threadIdx.y != 0) return;
     double mx = 0.0, rowsum = 0.0;
     if (r < h.n) {
         const double d = h.onsite ? h.onsite[r] : 0.0;
@@ -58,10 +77,7 @@ __global__ void __launch_bounds__(256) build_h_kernel(DevHam h) {
         mx = fabs(d);
         rowsum = fabs(d);
         for (int s = 0; s < h.zmax; ++s) {
-            const int64_t q = (int64_t)s * h.n + r;
-            const double2 acc = slot_value(h, q, h.field, h.nfield);
-            h.val[q] = acc;
-            const double a = habs(acc);
+            const double a = h.zmax <= kBuildLdsSlots ? mag[s * 64 + lane] : habs(h.val[(int64_t)s * h.n + r]);
             mx = fmax(mx, a);
             rowsum += a;
         }
@@ -75,40 +91,110 @@ __global__ void __launch_bounds__(256) build_h_kernel(DevHam h) {
         }
         if (h.ndict) h.drec[r] = make_double2(d, __longlong_as_double((long long)h.dpack[r]));
     }
-    // block maxima first: one device-scope atomic per block and quantity
-    red_mx[threadIdx.x] = mx;
-    red_rs[threadIdx.x] = rowsum;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) {
-            red_mx[threadIdx.x] = fmax(red_mx[threadIdx.x], red_mx[threadIdx.x + w]);
-            red_rs[threadIdx.x] = fmax(red_rs[threadIdx.x], red_rs[threadIdx.x + w]);
-        }
-        __syncthreads();
+    for (int off = 32; off > 0; off >>= 1) {
+        mx = fmax(mx, __shfl_xor(mx, off));
+        rowsum = fmax(rowsum, __shfl_xor(rowsum, off));
     }
-    // max over rows: nonnegative doubles order like their bit patterns
-    if (threadIdx.x == 0) {
-        atomicMax(&h.red[0], (unsigned long long)__double_as_longlong(red_mx[0]));
-        atomicMax(&h.red[1], (unsigned long long)__double_as_longlong(red_rs[0]));
+    if (lane == 0) {
+        h.hpart[blockIdx.x] = mx;
+        h.hpart[gridDim.x + blockIdx.x] = rowsum;
     }
 }
 
-// After build_h: the class table from each class's defining slot, and a
-// check that every slot holds its class's value (conjugated where marked);
-// any difference sets red[2], and the fused passes then read val instead.
-__global__ void __launch_bounds__(256) dict_check_kernel(DevHam h) {
-    const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (q < h.ndict) {
-        const int32_t rp = h.drep[q];
-        h.dval[q] = rp >= 0 ? h.val[rp] : make_double2(0.0, 0.0);
+// *flag |= bit if any lane sees bad: one atomic per wave (a field whose
+// bonds all differ sets the flag from every strip)
+__device__ __forceinline__ void raise_flag(unsigned long long *flag, bool bad, unsigned long long bit) {
+    const unsigned long long lanes = __ballot(bad);
+    if (lanes && (int)(threadIdx.x & 63) == __ffsll(lanes) - 1) atomicOr(flag, bit);
+}
+
+// After build_h, one thread per item: workgroup 0 reduces the partial maxima
+// (max |H_ij| into red[0], max row sum into red[1]); the others
+//   * value classes: the class table from each class's defining slot, and
+//     every slot against its class (conjugated where marked) -- a difference
+//     sets red[2], and the fused passes then read val instead;
+//   * strips: each strip thread's bond value per direction, every used bond
+//     of the strip against it bit for bit (else bit 0 of red[3]; bit 1 when an
+//     x bond is complex), and the diagonal in strip order.
+__global__ void __launch_bounds__(256) h_check_kernel(DevHam h, int64_t nparts) {
+    if (blockIdx.x == 0) {
+        __shared__ double red[2][256];
+        double m[2] = {0.0, 0.0};
+        for (int64_t b = threadIdx.x; b < nparts; b += 256) {
+            m[0] = fmax(m[0], h.hpart[b]);
+            m[1] = fmax(m[1], h.hpart[nparts + b]);
+        }
+        red[0][threadIdx.x] = m[0];
+        red[1][threadIdx.x] = m[1];
+        __syncthreads();
+        for (int w = 128; w > 0; w >>= 1) {
+            if (threadIdx.x < w)
+                for (int k = 0; k < 2; ++k) red[k][threadIdx.x] = fmax(red[k][threadIdx.x], red[k][threadIdx.x + w]);
+            __syncthreads();
+        }
+        if (threadIdx.x < 2) h.red[threadIdx.x] = (unsigned long long)__double_as_longlong(red[threadIdx.x][0]);
+        return;
     }
-    if (q >= (int64_t)h.zmax * h.n || h.col[q] < 0) return;
-    const int32_t cc = h.dcls[q];
-    const int32_t rp = h.drep[cc & 0x7ff];
-    double2 v = rp >= 0 ? h.val[rp] : make_double2(0.0, 0.0);
-    if (cc >> 15) v.y = -v.y;
-    const double2 w = h.val[q];
-    if (v.x != w.x || v.y != w.y) atomicOr(&h.red[2], 1ull);
+    const int64_t id = (blockIdx.x - 1) * (int64_t)256 + threadIdx.x;
+    const int64_t n = h.n;
+    if (h.ndict) {
+        if (id < h.ndict) {
+            const int32_t rp = h.drep[id];
+            h.dval[id] = rp >= 0 ? h.val[rp] : make_double2(0.0, 0.0);
+        }
+        if (id < (int64_t)h.zmax * n && h.col[id] >= 0) {
+            const int32_t cc = h.dcls[id];
+            const int32_t rp = h.drep[cc & 0x7ff];
+            double2 v = rp >= 0 ? h.val[rp] : make_double2(0.0, 0.0);
+            if (cc >> 15) v.y = -v.y;
+            const double2 w = h.val[id];
+            raise_flag(&h.red[2], v.x != w.x || v.y != w.y, 1ull);
+        }
+    }
+    const StripGeom &g = h.sg;
+    const int S = g.s;
+    if (S == 0 || id >= 5 * (int64_t)S * g.nt) return;
+    // item (d, m, strip thread): d = 4 the diagonal
+    const int d = (int)(id / ((int64_t)S * g.nt));
+    const int rem = (int)(id - (int64_t)d * S * g.nt);
+    const int m = rem / g.nt, tl = rem - m * g.nt;
+    const int x = tl % g.lx, k = tl / g.lx;
+    const int y0 = min(k * S, g.ly - S);
+    const int64_t i0 = (int64_t)x * g.ly + y0, i = i0 + m;
+    if (d == 4) {
+        h.sdiag[(int64_t)m * g.nt + tl] = h.diag[i];
+        return;
+    }
+    // the direction's first used bond of the strip (S >= 2), and this one
+    bool used;
+    int first = 0;
+    if (d == 0) {
+        used = m + 1 < S || y0 + S < g.ly || g.py;
+    } else if (d == 1) {
+        used = m > 0 || y0 > 0 || g.py;
+        first = y0 > 0 || g.py ? 0 : 1;
+    } else {
+        used = d == 2 ? (x + 1 < g.lx || g.px) : (x > 0 || g.px);
+    }
+    const bool any = d < 2 || used;
+    double2 u = make_double2(0.0, 0.0);
+    bool bad = false;
+    if (any) {
+        const int32_t q0 = h.sslot[d * n + i0 + first];
+        if (q0 >= 0) u = h.val[q0];
+        if (used) {
+            const int32_t q = h.sslot[d * n + i];
+            if (q < 0 || q0 < 0) {
+                bad = true;
+            } else {
+                const double2 v = h.val[q];
+                bad = v.x != u.x || v.y != u.y;
+            }
+        }
+    }
+    if (m == 0) h.stval[d * g.nt + tl] = u;
+    raise_flag(&h.red[3], bad, 1ull);
+    raise_flag(&h.red[3], d >= 2 && u.y != 0.0, 2ull);
 }
 
 __global__ void __launch_bounds__(256) slot_probe_kernel(DevHam h, const FieldComp *probe, int nprobe,
@@ -164,18 +250,13 @@ hipError_t launch_csc_gather(int64_t nbonds, int64_t n, const int64_t *kup, cons
 
 hipError_t launch_build_h(const DevHam &h, hipStream_t st) {
     if (h.n == 0) return hipSuccess;
-    hipError_t e = hipMemsetAsync(h.red, 0, 4 * sizeof(unsigned long long), st);
-    if (e != hipSuccess) return e;
-    const int bs = 256;
-    const int64_t nb = (h.n + bs - 1) / bs;
-    hipLaunchKernelGGL(build_h_kernel, dim3((unsigned)nb), dim3(bs), 0, st, h);
-    if (h.ndict) {
-        const int64_t work = std::max<int64_t>((int64_t)h.zmax * h.n, h.ndict);
-        hipLaunchKernelGGL(dict_check_kernel, dim3((unsigned)((work + bs - 1) / bs)), dim3(bs), 0, st, h);
-    }
-    e = hipGetLastError();
-    if (e == hipSuccess) e = launch_strip_check(h, st);
-    return e;
+    const int64_t nb = build_h_parts(h.n);
+    const int ny = std::max(1, std::min(h.zmax, 16));
+    hipLaunchKernelGGL(build_h_kernel, dim3((unsigned)nb), dim3(64, ny), h.zmax <= kBuildLdsSlots ? sizeof(double) * 64 * h.zmax : 0, st, h);
+    int64_t work = h.ndict ? std::max<int64_t>((int64_t)h.zmax * h.n, h.ndict) : 0;
+    if (h.sg.s > 0) work = std::max<int64_t>(work, 5 * (int64_t)h.sg.s * h.sg.nt);
+    hipLaunchKernelGGL(h_check_kernel, dim3((unsigned)(1 + (work + 255) / 256)), dim3(256), 0, st, h, nb);
+    return hipGetLastError();
 }
 
 hipError_t launch_slot_probe(const DevHam &h, const FieldComp *probe, int nprobe, double2 *out, hipStream_t st) {

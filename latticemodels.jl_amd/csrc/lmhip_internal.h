@@ -85,6 +85,7 @@ struct DevHam {
     // bit 0 when a strip's bonds of one direction differ, bit 1 when an x
     // bond is complex (strip kernel)
     unsigned long long *red = nullptr;
+    double *hpart = nullptr;    // [2][build_h_parts(n)] partial maxima of red[0] and red[1]
     // Value classes (zmax <= 4, n <= 10240): slots whose values are equal, or
     // conjugate, for every field amplitude share one class, so a fused pass
     // can read H's values from a table in LDS instead of from L2.  Per site a
@@ -123,6 +124,7 @@ struct DevHam {
 // kernels/launchers (hamiltonian.hip)
 // builds val/diag/rec (and drec/dval with the class check when h.ndict > 0)
 hipError_t launch_build_h(const DevHam &h, hipStream_t st);
+inline int64_t build_h_parts(int64_t n) { return (n + 63) / 64; }
 // CSC values of a fixed pattern -> bond amplitudes and on-site energies;
 // flag: bit 0 not Hermitian, bit 1 complex diagonal, bit 2 not finite
 hipError_t launch_csc_gather(int64_t nbonds, int64_t n, const int64_t *kup, const int64_t *klo, const int64_t *kd,
@@ -174,7 +176,6 @@ __host__ __device__ inline bool strip_coef_ok(const TaylorOut &o, bool xreal) {
 // strip kernel can run.  The per-strip check runs inside launch_build_h.
 bool strip_detect(const int32_t *col, int64_t n, int zmax, StripGeom *g, int32_t *sslot);
 int64_t strip_thread_count(const StripGeom &g);
-hipError_t launch_strip_check(const DevHam &h, hipStream_t st);
 // a strip polynomial waiting to be applied: the second side of a step whose
 // launch was deferred, with its H's strip values kept apart (the context's
 // are rebuilt by the next H)

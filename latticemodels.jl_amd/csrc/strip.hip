@@ -29,7 +29,7 @@
 //
 // Whether H qualifies is decided twice: the pattern on the host when the
 // geometry is set (strip_detect), and the values after every H build on the
-// device (strip_check_kernel: every used bond of a strip's direction equal
+// device (h_check_kernel: every used bond of a strip's direction equal
 // to the strip's value, bit for bit).  When either fails, the fused passes
 // run the general kernels of fused.hip, so this kernel changes speed, never
 // results.  Reference step: src/evolution.jl:73-78 (U P U' with U from
@@ -476,54 +476,6 @@ __global__ void __launch_bounds__(256) strip_snapshot_kernel(const double2 *__re
     if (blockIdx.x == 0 && threadIdx.x == 0) *coef_out = *coef;
 }
 
-// After build_h: each strip thread's bond value per direction (all used
-// bonds of the direction must agree bit for bit, else bit 0 of red[3]; bit 1
-// when an x bond is complex) and its diagonal in strip order.  One thread per
-// (direction, strip thread); the diagonal one per (position, strip thread).
-__global__ void __launch_bounds__(256) strip_check_kernel(DevHam h) {
-    const StripGeom &g = h.sg;
-    const int64_t idx = blockIdx.x * 256 + threadIdx.x;
-    const int S = g.s;
-    const int64_t n = h.n;
-    if (idx < 4 * g.nt) {
-        const int d = (int)(idx / g.nt), tl = (int)(idx - (int64_t)d * g.nt);
-        const int x = tl % g.lx, k = tl / g.lx;
-        const int y0 = min(k * S, g.ly - S);
-        bool bad = false, have = false;
-        double2 u = make_double2(0.0, 0.0);
-        for (int m = 0; m < S; ++m) {
-            bool used;
-            if (d == 0) used = m + 1 < S || y0 + S < g.ly || g.py;
-            else if (d == 1) used = m > 0 || y0 > 0 || g.py;
-            else if (d == 2) used = x + 1 < g.lx || g.px;
-            else used = x > 0 || g.px;
-            if (!used) continue;
-            const int64_t i = (int64_t)x * g.ly + y0 + m;
-            const int32_t q = h.sslot[d * n + i];
-            if (q < 0) {
-                bad = true;
-                continue;
-            }
-            const double2 v = h.val[q];
-            if (!have) {
-                u = v;
-                have = true;
-            } else if (v.x != u.x || v.y != u.y) {
-                bad = true;
-            }
-        }
-        h.stval[d * g.nt + tl] = u;
-        const bool xcomplex = d >= 2 && u.y != 0.0;
-        if (bad || xcomplex) atomicOr(&h.red[3], (bad ? 1ull : 0ull) | (xcomplex ? 2ull : 0ull));
-    }
-    for (int64_t e = idx; e < (int64_t)S * g.nt; e += (int64_t)gridDim.x * 256) {
-        const int m = (int)(e / g.nt), tl = (int)(e - (int64_t)m * g.nt);
-        const int x = tl % g.lx, k = tl / g.lx;
-        const int y0 = min(k * S, g.ly - S);
-        h.sdiag[e] = h.diag[(int64_t)x * g.ly + y0 + m];
-    }
-}
-
 template <int S, bool T, bool XR, bool TWO>
 const void *strip_fn() {
     return (const void *)strip_kernel<S, T, XR, TWO>;
@@ -666,13 +618,6 @@ bool strip_detect(const int32_t *col, int64_t n, int zmax, StripGeom *g, int32_t
 }
 
 int64_t strip_thread_count(const StripGeom &g) { return g.nt; }
-
-hipError_t launch_strip_check(const DevHam &h, hipStream_t st) {
-    if (h.sg.s == 0) return hipSuccess;
-    const int64_t work = (int64_t)std::max(4, h.sg.s) * h.sg.nt;
-    hipLaunchKernelGGL(strip_check_kernel, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, st, h);
-    return hipGetLastError();
-}
 
 namespace {
 
