@@ -301,10 +301,11 @@ int lmh_create(lmh_context **out, int device) {
     hipError_t e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     size_t free_b = 0;
     if (e == hipSuccess) e = hipMemGetInfo(&free_b, &ctx->mem_total);
-    if (e == hipSuccess) e = dalloc(&ctx->d_maxbits, lmh::kMaxTaylor);
-    if (e == hipSuccess) e = dalloc(&ctx->d_partmax, (size_t)lmh::taylor_order_scratch());
+    if (e == hipSuccess) e = dalloc(&ctx->d_masks, lmh::kTaylorMasks);
+    if (e == hipSuccess) e = hipMemsetAsync(ctx->d_masks, 0, sizeof(unsigned long long) * lmh::kTaylorMasks, ctx->stream);
     if (e == hipSuccess) e = dalloc(&ctx->d_overflow, 1);
-    if (e == hipSuccess) e = dalloc(&ctx->d_run, 1);
+    if (e == hipSuccess) e = hipMemsetAsync(ctx->d_overflow, 0, sizeof(int), ctx->stream);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&ctx->h_tout, sizeof(lmh::TaylorOut), 0);
     if (e == hipSuccess) e = dalloc(&ctx->d_tout, 1);
     if (e == hipSuccess) e = dalloc(&ctx->h.red, 4);
     if (e == hipSuccess) e = lmh::prepare_region_currents_static();
@@ -352,10 +353,8 @@ int lmh_destroy(lmh_context *ctx) {
     free_geometry(ctx->h);
     dfree(ctx->h.field);
     dfree(ctx->h.red);
-    dfree(ctx->d_maxbits);
-    dfree(ctx->d_partmax);
+    dfree(ctx->d_masks);
     dfree(ctx->d_overflow);
-    dfree(ctx->d_run);
     dfree(ctx->d_tout);
     dfree(ctx->d_rho);
     dfree(ctx->d_J);

@@ -680,6 +680,16 @@ int lmh_set_csc_values(lmh_context *ctx, int64_t nnz, const double *nzval) {
 }  // extern "C"
 namespace lmhapi {
 
+// the order search of the current dt, threshold and nztol at a table level
+hipError_t order_search(lmh_context *ctx, int level) {
+    hipError_t e = lmh::launch_taylor_order(ctx->h, ctx->dt, ctx->nztol, ctx->threshold, level, ctx->d_masks,
+                                            ctx->d_overflow, ctx->stream);
+    if (e == hipSuccess)
+        e = lmh::launch_taylor_finish(ctx->h.red, ctx->dt, ctx->threshold, ctx->d_masks, ctx->d_overflow, ctx->d_tout,
+                                      ctx->h_tout, ctx->stream);
+    return e;
+}
+
 // Takes up an order result: the larger neighbourhood tables when a column's
 // did not fit (one level at a time, each read back), then the value-class
 // and strip checks that travel with it, K and s.  An error leaves the solver
@@ -691,15 +701,10 @@ int order_finish(lmh_context *ctx, lmh::TaylorOut &out, int level0) {
         ++level;
         {
             ProfScope ps(ctx, LMH_KERNEL_TAYLOR_ORDER);
-            HIP_TRY(lmh::launch_taylor_order(h, ctx->dt, ctx->nztol, ctx->d_run, level, ctx->d_partmax,
-                                             ctx->d_maxbits, ctx->d_overflow, ctx->stream),
-                    "taylor_order launch");
-            HIP_TRY(lmh::launch_taylor_finish(h.red, ctx->d_run, ctx->d_maxbits, ctx->d_overflow, ctx->d_tout,
-                                              ctx->stream),
-                    "taylor finish launch");
+            HIP_TRY(order_search(ctx, level), "taylor_order launch");
         }
-        HIP_TRY(hipMemcpyAsync(&out, ctx->d_tout, sizeof out, hipMemcpyDeviceToHost, ctx->stream), "order readback");
         HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+        out = *ctx->h_tout;
     }
     if (!out.overflow) {
         ctx->order_level = level;
@@ -770,29 +775,19 @@ int lmh_update_solver(lmh_context *ctx, double dt, int force, double threshold, 
         // reductions, the per-column term maxima, K and the Horner
         // coefficients
         const int level0 = ctx->order_level_geom == ctx->geom_version + 1 ? ctx->order_level : 0;
-        {
-            ProfScope ps(ctx, LMH_KERNEL_TAYLOR_ORDER);
-            HIP_TRY(lmh::launch_taylor_setup(h.red, dt, threshold, ctx->d_run, ctx->d_overflow, ctx->stream),
-                    "taylor setup launch");
-            HIP_TRY(lmh::launch_taylor_order(h, dt, nztol, ctx->d_run, level0, ctx->d_partmax, ctx->d_maxbits,
-                                             ctx->d_overflow, ctx->stream),
-                    "taylor_order launch");
-            HIP_TRY(lmh::launch_taylor_finish(h.red, ctx->d_run, ctx->d_maxbits, ctx->d_overflow, ctx->d_tout,
-                                              ctx->stream),
-                    "taylor finish launch");
-        }
+        ctx->solver_ready = false;
         ctx->dt = dt;
         ctx->threshold = threshold;
         ctx->nztol = nztol;
+        {
+            ProfScope ps(ctx, LMH_KERNEL_TAYLOR_ORDER);
+            HIP_TRY(order_search(ctx, level0), "taylor_order launch");
+        }
         if (!K_out && !s_out && order_may_stay(ctx)) {
             // K stays on the device: the strip steps read it from there; the
             // result comes back behind an event and is taken up later
-            if (!ctx->h_tout) HIP_TRY(hipHostMalloc((void **)&ctx->h_tout, sizeof(lmh::TaylorOut), 0), "pinned result");
             if (!ctx->ev_order)
                 HIP_TRY(hipEventCreateWithFlags(&ctx->ev_order, hipEventDisableTiming), "hipEventCreate");
-            HIP_TRY(hipMemcpyAsync(ctx->h_tout, ctx->d_tout, sizeof(lmh::TaylorOut), hipMemcpyDeviceToHost,
-                                   ctx->stream),
-                    "order readback");
             HIP_TRY(hipEventRecord(ctx->ev_order, ctx->stream), "hipEventRecord");
             ctx->order_async = true;
             ctx->async_xreal = h.strip_xreal ? 1 : 0;
@@ -802,11 +797,10 @@ int lmh_update_solver(lmh_context *ctx, double dt, int force, double threshold, 
             ctx->solver_ready = true;
             return LMH_OK;
         }
-        // one readback of the result (with the reductions and the value-class
-        // / strip checks)
-        lmh::TaylorOut out;
-        HIP_TRY(hipMemcpyAsync(&out, ctx->d_tout, sizeof out, hipMemcpyDeviceToHost, ctx->stream), "order readback");
+        // the result (with the reductions and the value-class / strip checks)
+        // is in pinned memory once the search has run
         HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+        lmh::TaylorOut out = *ctx->h_tout;
         rc = order_finish(ctx, out, level0);
         if (rc) return rc;
         ctx->solver_version = ctx->param_version;

@@ -144,11 +144,9 @@ struct lmh_context {
     uint64_t solver_version = 0;
     uint64_t solver_serial = 0;       // bumped by every recompute of K, s and dt (lmh_update_solver)
     // scratch
-    unsigned long long *d_maxbits = nullptr;
-    double *d_partmax = nullptr;      // Taylor-order partial maxima per workgroup
+    unsigned long long *d_masks = nullptr;   // order search: terms above the threshold
     int *d_overflow = nullptr;
-    lmh::TaylorRun *d_run = nullptr;  // order-rule parameters derived on the device
-    lmh::TaylorOut *d_tout = nullptr; // its result, read back once per update
+    lmh::TaylorOut *d_tout = nullptr; // its result; the host's copy is h_tout
     double *d_rho = nullptr, *d_J = nullptr;
     double *d_hdiag = nullptr;
     double2 *d_hij = nullptr;
@@ -389,6 +387,7 @@ int state_settle(lmh_state *st);
 int ctx_settle_all(lmh_context *ctx);
 int state_normalize(lmh_state *st);
 void csc_release(lmh_context *ctx);
+hipError_t order_search(lmh_context *ctx, int level);
 int order_finish(lmh_context *ctx, lmh::TaylorOut &out, int level0);
 bool strip_step_path(const lmh_context *ctx);
 bool order_may_stay(const lmh_context *ctx);

@@ -135,21 +135,12 @@ hipError_t launch_slot_probe(const DevHam &h, const FieldComp *probe, int nprobe
 constexpr int kDictMaxClasses = 2048;
 constexpr int kDictMaxOffsets = 16;
 
-// The order rule's device records (taylor.hip).  TaylorRun is derived on the
-// device from H's reductions (red[0] max|H_ij|, red[1] max row abs-sum) by
-// launch_taylor_setup; the order kernels read it, and launch_taylor_finish
-// writes TaylorOut: the result with a copy of red[], and the Horner
-// coefficients of the step, so that a strip launch can take its term count
-// and coefficients from device memory instead of from the host.
+// The order rule's result (taylor.hip), written by launch_taylor_finish: with
+// a copy of red[], and the Horner coefficients of the step, so that a strip
+// launch can take its term count and coefficients from device memory instead
+// of from the host.
 constexpr int kStripMaxK = 31;          // Horner coefficients carried per polynomial
-struct TaylorRun {
-    double s, inv_s;            // s = nextpow(2, max|H| |dt|)
-    double thr;                 // threshold / s
-    double growth;              // |dt| rowsum / s: terms can only shrink from n + 1 > growth on
-    double dt;
-    int nmax;                   // first n with growth^n / n! <= thr (0: U = I)
-    int pad;
-};
+constexpr int kTaylorMasks = 64;        // words the search's workgroups report to
 struct TaylorOut {
     unsigned long long red[4];
     double s;
@@ -229,19 +220,17 @@ hipError_t strip_batch_table(const StripMemberDesc *m, int nm, void **d_args, in
 hipError_t launch_batched_strip(const void *d_args, const int64_t *d_ustart, int nm, int64_t nunits, size_t lds,
                                 bool tout, hipStream_t st);
 
-// kernels/launchers (taylor.hip): the reference's order rule on the device
-// (TaylorRun and TaylorOut are declared before the strip kernel's launchers).
-int taylor_order_levels();
-int64_t taylor_order_scratch();
-hipError_t launch_taylor_setup(const unsigned long long *red, double dt, double threshold, TaylorRun *run,
-                               int *overflow, hipStream_t st);
+// kernels/launchers (taylor.hip): the reference's order rule on the device.
 // level 0..taylor_order_levels()-1 picks the neighbourhood table size (the
-// grid-window kernel at level 0 when H is a grid stencil)
-hipError_t launch_taylor_order(const DevHam &h, double dt, double nztol, const TaylorRun *run, int level,
-                               double *partmax, unsigned long long *maxbits, int *overflow, hipStream_t st);
-hipError_t launch_taylor_finish(const unsigned long long *red, const TaylorRun *run,
-                                const unsigned long long *maxbits, const int *overflow, TaylorOut *out,
-                                hipStream_t st);
+// grid-window kernel at level 0 when H is a grid stencil); masks
+// (kTaylorMasks words) and overflow are clear before the search and left
+// clear by launch_taylor_finish, which writes the result to out (device) and
+// out_host (pinned).
+int taylor_order_levels();
+hipError_t launch_taylor_order(const DevHam &h, double dt, double nztol, double threshold, int level,
+                               unsigned long long *masks, int *overflow, hipStream_t st);
+hipError_t launch_taylor_finish(const unsigned long long *red, double dt, double threshold, unsigned long long *masks,
+                                int *overflow, TaylorOut *out, TaylorOut *out_host, hipStream_t st);
 
 // kernels/launchers (passes.hip)
 // lcols: columns swept per left-pass thread or block (0 = default); variant:
