@@ -285,7 +285,7 @@ struct lmh_kets {
         hipGraphExec_t exec;
     };
     std::vector<ChunkGraph> graphs;
-    const void *graph_basis = nullptr, *graph_lz = nullptr;
+    const void *graph_basis = nullptr, *graph_lz = nullptr, *graph_pin = nullptr;
     int graph_kd = 0;
     uint64_t graph_geom = 0;
     // host copies of the coefficients and basis lengths

@@ -218,20 +218,29 @@ int lmh_krylov_step(lmh_context *ctx, lmh_kets *k, double dt, int krylovdim, dou
                                                  S(jj + 1), ld, m, pre, pim, pw, d_alpha + (size_t)jj * m,
                                                  d_beta + (size_t)jj * m, st);
         };
+        // beta_jj, and the recurrence coefficients so far to the host: from
+        // the kernel for a few kets (8-byte writes over the link), else by a
+        // copy behind it
+        const bool direct = m <= 64;
+        auto norm = [&](int jj) {
+            return lmh::launch_lanczos_beta(pw, n, m, jj, d_alpha, d_beta, direct ? pin_abv : nullptr,
+                                            direct ? pin_abv + nalpha : nullptr, st);
+        };
         // the first chunk (start, `target` iterations, beta_target): replayed
         // from a graph when one was captured for this source buffer and length
         auto first_chunk = [&]() {
             hipError_t e = lmh::launch_lanczos_start(k->buf[src], n, ld, m, pw, st);
             for (int jj = 0; jj < target && e == hipSuccess; ++jj) e = iteration(jj);
-            if (e == hipSuccess) e = lmh::launch_lanczos_beta(pw, n, m, d_beta + (size_t)target * m, st);
+            if (e == hipSuccess) e = norm(target);
             return e;
         };
         if (ctx->krylov_graphs) {
-            if (k->graph_basis != k->basis || k->graph_lz != k->lz || k->graph_kd != kd ||
+            if (k->graph_basis != k->basis || k->graph_lz != k->lz || k->graph_pin != k->h_pin || k->graph_kd != kd ||
                 k->graph_geom != ctx->geom_version) {
                 krylov_graphs_free(k);
                 k->graph_basis = k->basis;
                 k->graph_lz = k->lz;
+                k->graph_pin = k->h_pin;
                 k->graph_kd = kd;
                 k->graph_geom = ctx->geom_version;
             }
@@ -271,10 +280,11 @@ int lmh_krylov_step(lmh_context *ctx, lmh_kets *k, double dt, int krylovdim, dou
                 ++mv;
                 beta_ready = false;
             }
-            if (!beta_ready) HIP_TRY(lmh::launch_lanczos_beta(pw, n, m, d_beta + (size_t)j * m, st), "Lanczos norm");
+            if (!beta_ready) HIP_TRY(norm(j), "Lanczos norm");
             beta_ready = false;
-            HIP_TRY(hipMemcpyAsync(pin_abv, d_alpha, 8 * (nalpha + (size_t)(j + 1) * m), hipMemcpyDeviceToHost, st),
-                    "Lanczos readback");
+            if (!direct)
+                HIP_TRY(hipMemcpyAsync(pin_abv, d_alpha, 8 * (nalpha + (size_t)(j + 1) * m), hipMemcpyDeviceToHost, st),
+                        "Lanczos readback");
             HIP_TRY(hipStreamSynchronize(st), "hipStreamSynchronize");
             bool open = false;
             for (int64_t c = 0; c < m; ++c) {
@@ -328,16 +338,21 @@ int lmh_krylov_step(lmh_context *ctx, lmh_kets *k, double dt, int krylovdim, dou
             longest = std::max(longest, len[c]);
         }
         k->krylov_len = longest;
-        // through the pinned staging (its previous uploads ended before the
-        // wait above)
-        std::memcpy(pin_coefv, coef.data(), sizeof(double2) * (size_t)m * kd);
-        std::memcpy(pin_lenv, len.data(), sizeof(int) * (size_t)m);
-        HIP_TRY(hipMemcpyAsync(k->coef, pin_coefv, sizeof(double2) * (size_t)m * kd, hipMemcpyHostToDevice, st),
-                "Krylov coefficient upload");
-        HIP_TRY(hipMemcpyAsync(k->len, pin_lenv, sizeof(int) * (size_t)m, hipMemcpyHostToDevice, st),
-                "Krylov coefficient upload");
         const int dst = (src + 1) % 3;
-        {
+        if (m == 1 && len[0] > 0 && len[0] <= lmh::kCombineArgs) {
+            ProfScope ps(ctx, LMH_KERNEL_KRYLOV);
+            HIP_TRY(lmh::launch_krylov_combine_one(k->basis, vstride, reinterpret_cast<const double *>(coef.data()),
+                                                   len[0], k->buf[dst], n, st),
+                    "Krylov combine");
+        } else {
+            // through the pinned staging (its previous uploads ended before
+            // the wait above)
+            std::memcpy(pin_coefv, coef.data(), sizeof(double2) * (size_t)m * kd);
+            std::memcpy(pin_lenv, len.data(), sizeof(int) * (size_t)m);
+            HIP_TRY(hipMemcpyAsync(k->coef, pin_coefv, sizeof(double2) * (size_t)m * kd, hipMemcpyHostToDevice, st),
+                    "Krylov coefficient upload");
+            HIP_TRY(hipMemcpyAsync(k->len, pin_lenv, sizeof(int) * (size_t)m, hipMemcpyHostToDevice, st),
+                    "Krylov coefficient upload");
             ProfScope ps(ctx, LMH_KERNEL_KRYLOV);
             HIP_TRY(lmh::launch_krylov_combine(k->basis, vstride, k->coef, kd, k->len, k->buf[src], k->buf[dst], n, ld,
                                                m, st),

@@ -21,101 +21,135 @@ namespace {
 
 constexpr int kLzThreads = 256;
 
-__device__ __forceinline__ double block_sum(double v, double *red) {
-    const int t = threadIdx.x;
-    red[t] = v;
+constexpr int kLzWaves = kLzThreads / 64;
+
+// block sums of R values at once, in every thread (fixed order): shuffles
+// within a wavefront, one barrier for the wavefronts' sums.  `red` holds
+// kLzWaves * R doubles and is not used again before the next barrier.
+template <int R>
+__device__ __forceinline__ void block_sums(double (&v)[R], double *red) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] += __shfl_xor(v[r], off);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int r = 0; r < R; ++r) red[(threadIdx.x >> 6) * R + r] = v[r];
     __syncthreads();
-    for (int w = kLzThreads / 2; w > 0; w >>= 1) {
-        if (t < w) red[t] += red[t + w];
-        __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        v[r] = red[r];
+#pragma unroll
+        for (int w = 1; w < kLzWaves; ++w) v[r] += red[w * R + r];
     }
-    const double r = red[0];
-    __syncthreads();
-    return r;
 }
 
-// sum of a column's nb partials, by the whole block (fixed order)
-__device__ __forceinline__ double column_total(const double *part, int nb, double *red) {
-    double acc = 0.0;
-    for (int b = threadIdx.x; b < nb; b += kLzThreads) acc += part[b];
-    return block_sum(acc, red);
+// a thread's share of a column's nb partials (fixed order)
+__device__ __forceinline__ double partial_share(const double *part, int nb) {
+    const int t = threadIdx.x;
+    double acc = t < nb ? part[t] : 0.0;
+    for (int b = t + kLzThreads; b < nb; b += kLzThreads) acc += part[b];
+    return acc;
 }
 
 // v_1 = psi / |psi| for every column: partial |psi|^2 per block
 __global__ void __launch_bounds__(kLzThreads) lanczos_norm_kernel(const double2 *__restrict__ X, int64_t n, int64_t ld,
                                                                  double *__restrict__ part, int nb) {
-    __shared__ double red[kLzThreads];
+    __shared__ double red[kLzWaves];
     const int64_t c = blockIdx.y;
     const int64_t i = (int64_t)blockIdx.x * kLzThreads + threadIdx.x;
-    double s = 0.0;
+    double s[1] = {0.0};
     if (i < n) {
         const double2 v = X[c * ld + i];
-        s = v.x * v.x + v.y * v.y;
+        s[0] = v.x * v.x + v.y * v.y;
     }
-    s = block_sum(s, red);
-    if (threadIdx.x == 0) part[c * nb + blockIdx.x] = s;
+    block_sums(s, red);
+    if (threadIdx.x == 0) part[c * nb + blockIdx.x] = s[0];
 }
 
-// beta[c] = |w| from the column's partials of |w|^2 (one block per column)
-__global__ void __launch_bounds__(kLzThreads) lanczos_beta_kernel(const double *__restrict__ part, int nb,
-                                                                 double *__restrict__ beta_out) {
-    __shared__ double red[kLzThreads];
+// beta_j[c] = |w_j| from the column's partials of |w|^2 (one block per column).
+// With ab_host the block also writes the column's alpha_0 .. alpha_{j-1} and
+// beta_0 .. beta_j to the host's pinned copy: a copy after the kernel costs
+// ~5 us and a gap of its own.
+__global__ void __launch_bounds__(kLzThreads) lanczos_beta_kernel(const double *__restrict__ part, int nb, int64_t m, int j,
+                                                                 const double *__restrict__ alpha, double *__restrict__ beta,
+                                                                 double *__restrict__ alpha_host,
+                                                                 double *__restrict__ beta_host) {
+    __shared__ double red[kLzWaves];
     const int64_t c = blockIdx.x;
-    const double b = sqrt(column_total(part + c * nb, nb, red));
-    if (threadIdx.x == 0) beta_out[c] = b;
+    double b[1] = {partial_share(part + c * nb, nb)};
+    block_sums(b, red);
+    const double bj = sqrt(b[0]);
+    if (threadIdx.x == 0) beta[j * m + c] = bj;
+    if (!alpha_host) return;
+    for (int q = threadIdx.x; q <= j; q += kLzThreads) {
+        if (q < j) alpha_host[q * m + c] = alpha[q * m + c];
+        beta_host[q * m + c] = q < j ? beta[q * m + c] : bj;
+    }
 }
 
 // beta_j = |W| (partials part_w); v_j = W / beta_j into Vj (0 stays 0), block 0
-// recording beta_j; Wn = H v_j - beta_j v_{j-1}; partials of <v_j, Wn>
+// recording beta_j; Wn = H v_j - beta_j v_{j-1}; partials of <v_j, Wn>.
+// Bound by latency (N = 10^5: 16 MB through L2 and 392 workgroups): H W is
+// formed unscaled, so its loads and gathers run while the norm is summed.
+// With LDS tree sums (8 barriers each, three sums) and the loads behind the
+// first of them 7.7 us, now 6.1; the kernel below 5.4, now 3.6 (N = 100352,
+// 3 neighbours, one column).
 template <int ZR>
 __global__ void __launch_bounds__(kLzThreads) lanczos_matvec_kernel(
     const int32_t *__restrict__ col, const double2 *__restrict__ val, const double *__restrict__ diag, int64_t n,
     int zmax, const double2 *__restrict__ W, const double *__restrict__ part_w, double2 *__restrict__ Vj,
     const double2 *__restrict__ Vprev, double2 *__restrict__ Wn, int64_t ld, double *__restrict__ beta_out,
     double *__restrict__ part_re, double *__restrict__ part_im, int nb) {
-    __shared__ double red[kLzThreads];
+    __shared__ double red[kLzWaves], red2[2 * kLzWaves];
     const int64_t c = blockIdx.y;
-    const double b = sqrt(column_total(part_w + c * nb, nb, red));
-    const double inv = b > 0.0 ? 1.0 / b : 0.0;
     const int64_t i = (int64_t)blockIdx.x * kLzThreads + threadIdx.x;
-    double dre = 0.0, dim = 0.0;
-    if (i < n) {
-        const double2 *w = W + c * ld;
-        const double2 wi = w[i];
-        const double2 vi = make_double2(wi.x * inv, wi.y * inv);
-        Vj[c * ld + i] = vi;
-        const double d = diag[i];
-        double2 hw = make_double2(d * wi.x, d * wi.y);
+    const bool on = i < n;
+    const int64_t ic = on ? i : n - 1;
+    const double2 *w = W + c * ld;
+    int32_t cq[ZR];
+    double2 hv[ZR];
 #pragma unroll
-        for (int q = 0; q < ZR; ++q) {
-            if (q < zmax) {
-                const int32_t cq = col[(int64_t)q * n + i];
-                if (cq >= 0) {
-                    const double2 hv = val[(int64_t)q * n + i];
-                    const double2 x = w[cq];
-                    hw.x += hv.x * x.x - hv.y * x.y;
-                    hw.y += hv.x * x.y + hv.y * x.x;
-                }
-            }
+    for (int q = 0; q < ZR; ++q) {
+        cq[q] = q < zmax ? col[(int64_t)q * n + ic] : -1;
+        if (ZR <= 9 && q < zmax) hv[q] = val[(int64_t)q * n + ic];
+    }
+    double b[1] = {partial_share(part_w + c * nb, nb)};
+    const double2 wi = w[ic];
+    const double d = diag[ic];
+    double2 p = make_double2(0.0, 0.0);
+    if (Vprev) p = Vprev[c * ld + ic];
+    double2 hw = make_double2(d * wi.x, d * wi.y);
+#pragma unroll
+    for (int q = 0; q < ZR; ++q)
+        if (cq[q] >= 0) {
+            const double2 h = ZR <= 9 ? hv[q] : val[(int64_t)q * n + ic];
+            const double2 x = w[cq[q]];
+            hw.x += h.x * x.x - h.y * x.y;
+            hw.y += h.x * x.y + h.y * x.x;
         }
+    block_sums(b, red);
+    const double beta = sqrt(b[0]);
+    const double inv = beta > 0.0 ? 1.0 / beta : 0.0;
+    double dot[2] = {0.0, 0.0};                          // conj(v_i) r
+    if (on) {
+        const double2 vi = make_double2(wi.x * inv, wi.y * inv);
         double2 r = make_double2(hw.x * inv, hw.y * inv);       // H v_j
         if (Vprev) {
-            const double2 p = Vprev[c * ld + i];
-            r.x -= b * p.x;
-            r.y -= b * p.y;
+            r.x -= beta * p.x;
+            r.y -= beta * p.y;
         }
+        Vj[c * ld + i] = vi;
         Wn[c * ld + i] = r;
-        // conj(v_i) r
-        dre = vi.x * r.x + vi.y * r.y;
-        dim = vi.x * r.y - vi.y * r.x;
+        dot[0] = vi.x * r.x + vi.y * r.y;
+        dot[1] = vi.x * r.y - vi.y * r.x;
     }
-    dre = block_sum(dre, red);
-    dim = block_sum(dim, red);
+    block_sums(dot, red2);
     if (threadIdx.x == 0) {
-        part_re[c * nb + blockIdx.x] = dre;
-        part_im[c * nb + blockIdx.x] = dim;
+        part_re[c * nb + blockIdx.x] = dot[0];
+        part_im[c * nb + blockIdx.x] = dot[1];
+        if (blockIdx.x == 0) beta_out[c] = beta;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) beta_out[c] = b;
 }
 
 // alpha = <v_j, W> from the partials; W -= alpha v_j; partials of |W|^2; block
@@ -125,23 +159,26 @@ __global__ void __launch_bounds__(kLzThreads) lanczos_orth_kernel(const double2 
                                                                  const double *__restrict__ part_im, int nb,
                                                                  double *__restrict__ alpha_out,
                                                                  double *__restrict__ part_nrm) {
-    __shared__ double red[kLzThreads];
+    __shared__ double red[2 * kLzWaves], red2[kLzWaves];
     const int64_t c = blockIdx.y;
-    const double are = column_total(part_re + c * nb, nb, red);
-    const double aim = column_total(part_im + c * nb, nb, red);
     const int64_t i = (int64_t)blockIdx.x * kLzThreads + threadIdx.x;
-    double s = 0.0;
+    const int64_t ic = i < n ? i : n - 1;
+    const double2 v = Vj[c * ld + ic];
+    double2 w = W[c * ld + ic];
+    double a[2] = {partial_share(part_re + c * nb, nb), partial_share(part_im + c * nb, nb)};
+    block_sums(a, red);
+    double s[1] = {0.0};
     if (i < n) {
-        const double2 v = Vj[c * ld + i];
-        double2 w = W[c * ld + i];
-        w.x -= are * v.x - aim * v.y;
-        w.y -= are * v.y + aim * v.x;
+        w.x -= a[0] * v.x - a[1] * v.y;
+        w.y -= a[0] * v.y + a[1] * v.x;
         W[c * ld + i] = w;
-        s = w.x * w.x + w.y * w.y;
+        s[0] = w.x * w.x + w.y * w.y;
     }
-    s = block_sum(s, red);
-    if (threadIdx.x == 0) part_nrm[c * nb + blockIdx.x] = s;
-    if (blockIdx.x == 0 && threadIdx.x == 0) alpha_out[c] = are;
+    block_sums(s, red2);
+    if (threadIdx.x == 0) {
+        part_nrm[c * nb + blockIdx.x] = s[0];
+        if (blockIdx.x == 0) alpha_out[c] = a[0];
+    }
 }
 
 // Y[:, c] = sum_{k < len[c]} coef[c][k] V_k[:, c]; len[c] < 0: a copy of X[:, c]
@@ -166,6 +203,26 @@ __global__ void __launch_bounds__(kLzThreads) krylov_combine_kernel(const double
         acc.y += a.x * v.y + a.y * v.x;
     }
     Y[c * ld + i] = acc;
+}
+
+// the same for one ket whose coefficients fit the kernel's arguments: no
+// upload in front of it (two copies of ~5 us)
+struct CombineCoef {
+    double2 a[kCombineArgs];
+};
+__global__ void __launch_bounds__(kLzThreads) krylov_combine_one_kernel(const double2 *__restrict__ V, int64_t vstride,
+                                                                       CombineCoef coef, int L, double2 *__restrict__ Y,
+                                                                       int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * kLzThreads + threadIdx.x;
+    if (i >= n) return;
+    double2 acc = make_double2(0.0, 0.0);
+    for (int k = 0; k < L; ++k) {
+        const double2 a = coef.a[k];
+        const double2 v = V[k * vstride + i];
+        acc.x += a.x * v.x - a.y * v.y;
+        acc.y += a.x * v.y + a.y * v.x;
+    }
+    Y[i] = acc;
 }
 
 }  // namespace
@@ -203,9 +260,20 @@ hipError_t launch_lanczos_iteration(const DevHam &h, const double2 *W, const dou
     return hipGetLastError();
 }
 
-hipError_t launch_lanczos_beta(const double *part, int64_t n, int64_t m, double *beta_out, hipStream_t st) {
-    hipLaunchKernelGGL(lanczos_beta_kernel, dim3((unsigned)m), dim3(kLzThreads), 0, st, part, lanczos_blocks(n),
-                       beta_out);
+hipError_t launch_lanczos_beta(const double *part, int64_t n, int64_t m, int j, const double *alpha, double *beta,
+                               double *alpha_host, double *beta_host, hipStream_t st) {
+    hipLaunchKernelGGL(lanczos_beta_kernel, dim3((unsigned)m), dim3(kLzThreads), 0, st, part, lanczos_blocks(n), m, j,
+                       alpha, beta, alpha_host, beta_host);
+    return hipGetLastError();
+}
+
+hipError_t launch_krylov_combine_one(const double2 *V, int64_t vstride, const double *coef, int len, double2 *Y,
+                                     int64_t n, hipStream_t st) {
+    if (len < 0 || len > kCombineArgs) return hipErrorInvalidValue;
+    CombineCoef cf{};
+    for (int k = 0; k < len; ++k) cf.a[k] = make_double2(coef[2 * k], coef[2 * k + 1]);
+    hipLaunchKernelGGL(krylov_combine_one_kernel, dim3((unsigned)lanczos_blocks(n)), dim3(kLzThreads), 0, st, V, vstride,
+                       cf, len, Y, n);
     return hipGetLastError();
 }
 

@@ -294,8 +294,15 @@ hipError_t launch_lanczos_iteration(const DevHam &h, const double2 *W, const dou
                                     const double2 *Vprev, double2 *Wn, int64_t ld, int64_t m, double *part_re,
                                     double *part_im, double *part_wn, double *alpha_out, double *beta_out,
                                     hipStream_t st);
-// beta_out[c] = sqrt(sum of column c's partials)
-hipError_t launch_lanczos_beta(const double *part, int64_t n, int64_t m, double *beta_out, hipStream_t st);
+// beta_j of every column (beta + j m) from its partials; with alpha_host /
+// beta_host (pinned, the layout of alpha / beta) indices 0 .. j to the host too
+hipError_t launch_lanczos_beta(const double *part, int64_t n, int64_t m, int j, const double *alpha, double *beta,
+                               double *alpha_host, double *beta_host, hipStream_t st);
+// Y = sum_{k < len} coef[k] V_k of one ket, coef (re, im pairs, host memory)
+// carried as kernel arguments
+constexpr int kCombineArgs = 64;
+hipError_t launch_krylov_combine_one(const double2 *V, int64_t vstride, const double *coef, int len, double2 *Y,
+                                     int64_t n, hipStream_t st);
 // Y[:, c] = sum_k coef[c * kmax + k] V_k[:, c] for k < len[c]; len[c] < 0: Y[:, c] = X[:, c]
 hipError_t launch_krylov_combine(const double2 *V, int64_t vstride, const double2 *coef, int kmax, const int *len,
                                  const double2 *X, double2 *Y, int64_t n, int64_t ld, int64_t m, hipStream_t st);
