@@ -189,6 +189,13 @@ __global__ void __launch_bounds__(256) h_check_kernel(DevHam h, int64_t nparts) 
             } else {
                 const double2 v = h.val[q];
                 bad = v.x != u.x || v.y != u.y;
+                // (the kernel takes the bonds of one side of a site as the
+                // conjugates of its neighbour's)
+                const int32_t qc = d == 1 ? h.sslot[i0] : (d == 3 && x > 0 ? h.sslot[2 * n + i - g.ly] : -1);
+                if (qc >= 0) {
+                    const double2 w = h.val[qc];
+                    bad = bad || v.x != w.x || v.y != -w.y;
+                }
             }
         }
     }

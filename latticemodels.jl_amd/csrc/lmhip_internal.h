@@ -38,18 +38,22 @@ struct FieldComp {
 // Grid-stencil geometry of H for the strip kernel (strip.hip): site
 // i = x * ly + y on an lx x ly grid, every stored entry of a row being the
 // diagonal or one of the four grid neighbours (y +- 1, x +- 1; across the
-// edges when px / py).  A thread owns a strip of s consecutive sites of one
-// x column (y0 .. y0 + s - 1; the last strip of a column overlaps its
-// neighbour when s does not divide ly), a workgroup `cols` columns of P.
+// edges when px / py).  A strip is s consecutive sites of one x column
+// (y0 .. y0 + s - 1), a thread owns the strips of bx neighbouring x columns
+// (the last strip or block overlaps its neighbour when s does not divide ly,
+// or bx lx), a workgroup `cols` columns of P.
 struct StripGeom {
     int lx = 0, ly = 0;
-    int lyp = 0;                // LDS length of an x column (ly rounded up to odd)
+    int lyp = 0;                // LDS length of bx x columns (bx * ly rounded up to odd)
     int px = 0, py = 0;         // periodic along x / y
     int s = 0;                  // sites per strip (0: H is not a grid stencil)
+    int bx = 0;                 // x columns per thread
     int q = 0;                  // strips per x column
-    int nt = 0;                 // threads per column of P = lx * q
+    int nt = 0;                 // strips of a column of P = lx * q (strip k of x column x: k * lx + x)
+    int nthr = 0;               // threads per column of P
+    int threads = 0;            // workgroup size
     int cols = 0;               // columns of P per workgroup
-    int region = 0;             // LDS entries per column: lx * lyp + 1 (the last holds 0)
+    int region = 0;             // LDS entries per column (the last holds 0)
 };
 
 // Geometry + Hamiltonian in ELL layout on the device.
@@ -166,7 +170,6 @@ __host__ __device__ inline bool strip_coef_ok(const TaylorOut &o, bool xreal) {
 // direction ([4][n]); false when H's pattern is not a grid stencil the
 // strip kernel can run.  The per-strip check runs inside launch_build_h.
 bool strip_detect(const int32_t *col, int64_t n, int zmax, StripGeom *g, int32_t *sslot);
-int64_t strip_thread_count(const StripGeom &g);
 // a strip polynomial waiting to be applied: the second side of a step whose
 // launch was deferred, with its H's strip values kept apart (the context's
 // are rebuilt by the next H)

@@ -9,22 +9,30 @@
 // every bond of one direction has the same value.  This kernel uses both
 // facts:
 //
-//   * a thread owns a strip of S consecutive sites (x, y0 .. y0+S-1) of a
-//     column of P and keeps y and x of the Horner recursion in registers; the
-//     y +- 1 neighbours are its own registers (the strip ends read one value
-//     of the neighbouring strip), so per site and term only the two x +- 1
-//     neighbours come from LDS, plus one write of the site's new value;
-//   * the four bond values of a strip are four complex registers, read once
-//     per launch; the diagonal (on-site disorder) is streamed from L2, six
-//     sites ahead.
+//   * a thread owns a block of BX x columns by S sites of a column of P and
+//     keeps y and x of the Horner recursion in registers; neighbours inside
+//     the block are its own registers, so per term only the sites around the
+//     block come from LDS, plus one write of each site on its edge;
+//   * the block's bond values are registers, read once per launch; so is the
+//     diagonal (on-site disorder) of a small block, a large one streams it
+//     from L2 a row ahead.
 //
-// Per Horner term  y <- x + (-i dt / (s k)) H y  the new values of a column
-// are written to its LDS copy (one x column per ly-rounded-to-odd run, so the
-// x +- 1 reads of a wave's consecutive lanes hit distinct banks), a barrier,
-// then every thread reads its two neighbour strips and updates its sites.
-// The column is loaded with gfx950 direct-to-LDS loads (global_load_lds
-// 16 B per lane), which keeps 160 KB per CU in flight without VGPRs: one
-// workgroup per CU loads at the HBM rate that a plain read kernel reaches.
+// Per Horner term  y <- x + (-i dt / (s k)) H y  the new values of a block's
+// edge are published to the column's LDS copy.  Where S divides ly a term
+// runs in two phases of rows, each phase's values being published while the
+// other computes (a write costs the LDS as much as three reads: published on
+// their own before the term, they took a third of it); else the values are
+// published, then a term runs (rows that two blocks share would belong to
+// different phases).  The column is loaded with gfx950 direct-to-LDS loads
+// (global_load_lds 16 B per lane).  A workgroup has as few wavefronts as a
+// column needs: 8 wavefronts a CU, in one workgroup at N = 10^4, whose loads
+// and stores then only overlap with other CUs' sums, in several at smaller N.
+// A step's launch (both sides, K = 8), strips of one column by 12 .. 20 sites
+// in workgroups of 512 before, blocks now: N = 100 48 -> 21 us, 851 47 -> 30,
+// 1681 144 -> 89, 2304 165 -> 143, 4096 518 -> 491, 6400 1374 -> 1182, 10^4
+// 2866 -> 2252.  At N = 10^4 a term takes 4400 cycles per CU (7200 before), of
+// which FP64 issue 3020 and LDS 3090; loads and stores take 1.0 ms of the
+// launch, 0.68 at the copy rate.
 // The workgroup is persistent over its share of the columns.
 //
 // Whether H qualifies is decided twice: the pattern on the host when the
@@ -48,12 +56,23 @@ namespace lmh {
 
 namespace {
 
-constexpr int kStripThreads = 512;      // 8 waves, 256 VGPRs each: one workgroup per CU
+constexpr int kStripThreads = 512;      // 8 waves of 256 VGPRs per CU: one workgroup of 512, ..., eight of 64
 constexpr int kStripLdsBytes = 163840;
 constexpr int kStripMaxN = 10240;
-constexpr int kDiagAhead = 6;           // diagonal loads in flight ahead of their site
-constexpr int kLdsAhead = 2;            // neighbour-strip reads ahead of their site
-constexpr int kStripS[] = {4, 6, 8, 10, 12, 16, 18, 20};
+// blocks of x columns by sites: B(bx, s)
+#define LMH_STRIP_SHAPES(B) B(1, 20) B(2, 10) B(2, 8) B(2, 6) B(2, 4) B(4, 4)
+struct StripShape {
+    int bx, s;
+};
+constexpr StripShape kStripShapes[] = {
+#define LMH_STRIP_SHAPE(BX, S) {BX, S},
+    LMH_STRIP_SHAPES(LMH_STRIP_SHAPE)
+#undef LMH_STRIP_SHAPE
+};
+constexpr int strip_shape_id(int bx, int s) { return bx * 32 + s; }
+// a block with inner sites does not publish them: its neighbours must not
+// read them, so blocks may not overlap nor end early
+constexpr bool strip_whole(int bx, int s) { return bx > 2 && s > 2; }
 // (kStripMaxK: Horner coefficients passed with the launch or read from a
 // TaylorOut, lmhip_internal.h)
 
@@ -71,6 +90,13 @@ struct StripPoly {
 // a device TaylorOut read through the constant address space: wave-uniform
 // scalar loads (nothing writes it while a strip launch runs)
 typedef __attribute__((address_space(4))) const TaylorOut ConstTaylorOut;
+
+// global memory by pointers read from memory (a batch member's): told apart
+// from LDS, whose counter their loads and stores would otherwise hold up
+typedef double vec2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(1))) vec2 GlobalVec2;
+typedef __attribute__((address_space(1))) const vec2 ConstGlobalVec2;
+typedef __attribute__((address_space(1))) const double ConstGlobalDouble;
 
 struct StripArgs {
     StripGeom g;
@@ -103,26 +129,37 @@ __device__ __forceinline__ int64_t strip_xcd_order(int64_t b, int64_t nprog) {
     return (b % kNumXCD) * per + b / kNumXCD;
 }
 
+// LDS place of x column x of a column of P: bx x columns to a run of pitch
+// lyp (odd, so that the lanes of a wave, whose blocks sit a run apart, read
+// from distinct banks)
+__device__ __forceinline__ int strip_run(const StripGeom &g, int x) {
+    const int r = x / g.bx;
+    return r * g.lyp + (x - r * g.bx) * g.ly;
+}
+
 // direct-to-LDS loads of the column group starting at jb: one wave
-// instruction per 64-site chunk of an x column
+// instruction per 64 sites of a run
 __device__ __forceinline__ void strip_dma(const StripArgs &a, double2 *lds, int64_t jb, int wave, int lane) {
     const StripGeom &g = a.g;
     int64_t ldg = a.ld;
     asm volatile("" : "+s"(ldg));
-    const int nch = (g.ly + 63) >> 6;
-    const int per_col = g.lx * nch;
+    const int len = g.bx * g.ly;
+    const int nch = (len + 63) >> 6, nrun = (g.lx + g.bx - 1) / g.bx;
+    const int per_col = nrun * nch;
     const int npair = g.cols * per_col;
-    for (int p = wave; p < npair; p += kStripThreads / 64) {
+    const int waves = (int)blockDim.x >> 6;
+    for (int p = wave; p < npair; p += waves) {
         const int gg = p / per_col;
         const int rem = p - gg * per_col;
-        const int xc = rem / nch, ch = rem - xc * nch;
+        const int r = rem / nch, ch = rem - r * nch;
         const int64_t jj = jb + gg;
-        const int y = ch * 64 + lane;
-        if (jj < a.ncols && y < g.ly) {
-            const double2 *src = a.X + jj * ldg + (int64_t)xc * g.ly + y;
+        const int e = ch * 64 + lane;
+        const int i = r * len + e;
+        if (jj < a.ncols && e < len && i < a.n) {
+            const double2 *src = a.X + jj * ldg + i;
             __builtin_amdgcn_global_load_lds(
                 (const void *)src,
-                (__attribute__((address_space(3))) void *)(lds + gg * g.region + xc * g.lyp + ch * 64), 16, 0, 0);
+                (__attribute__((address_space(3))) void *)(lds + gg * g.region + r * g.lyp + ch * 64), 16, 0, 0);
         }
     }
 }
@@ -133,17 +170,22 @@ __device__ __forceinline__ void strip_store(const StripArgs &a, const double2 *l
     const StripGeom &g = a.g;
     int64_t ldg = a.ld;
     asm volatile("" : "+s"(ldg));
-    const int nch = (g.ly + 63) >> 6;
-    const int per_col = g.lx * nch;
+    const int len = g.bx * g.ly;
+    const int nch = (len + 63) >> 6, nrun = (g.lx + g.bx - 1) / g.bx;
+    const int per_col = nrun * nch;
     const int npair = g.cols * per_col;
-    for (int p = wave; p < npair; p += kStripThreads / 64) {
+    const int waves = (int)blockDim.x >> 6;
+    for (int p = wave; p < npair; p += waves) {
         const int gg = p / per_col;
         const int rem = p - gg * per_col;
-        const int xc = rem / nch, ch = rem - xc * nch;
+        const int r = rem / nch, ch = rem - r * nch;
         const int64_t jj = jb + gg;
-        const int y = ch * 64 + lane;
-        if (jj < a.ncols && y < g.ly)
-            a.Y[jj * ldg + (int64_t)xc * g.ly + y] = lds[gg * g.region + xc * g.lyp + y];
+        const int e = ch * 64 + lane;
+        const int i = r * len + e;
+        if (jj < a.ncols && e < len && i < a.n) {
+            const double2 v = lds[gg * g.region + r * g.lyp + e];
+            ((GlobalVec2 *)a.Y)[jj * ldg + i] = vec2{v.x, v.y};
+        }
     }
 }
 
@@ -158,75 +200,98 @@ __device__ __forceinline__ void hmac(double2 &acc, double2 h, double2 v) {
     }
 }
 
-// One column group of a strip pass, its columns already in LDS (with the
-// zero slot set).  TOUT: the result is written conjugate-transposed
-// (Y[s, j] = conj(y_s)), else plainly; XR: the x bonds are real (Landau
-// gauge, no field).  At the end the next group (na, njb, when next) is
-// loaded into LDS with its zero slot, ready for the next call.
-// a thread's place in the column group: its strip, its neighbour strips'
-// LDS positions and its bond values
+constexpr int kNoSite = 1 << 30;
+
+// A thread's place in the column group: its block of BX x columns by S sites
+// and the LDS positions of its columns and neighbours.
+template <int BX>
 struct StripThread {
-    int slot, tl, x, y0, skip, base, xp, xm, lo, hi;
+    int slot, tl, x0, y0, skx, sky;              // skx, sky: columns and rows shared with the block before
+    int cb[BX], xl, xr;                          // own columns at y0; the columns left and right of the block
+    int lo, hi;                                  // from cb: the sites below and above the block (kNoSite: absent)
+    int zero;                                    // an entry that holds 0
     bool act;
-    double2 hyp, hym, hxp, hxm;                  // BONDS: the first polynomial's bond values
 };
 
-template <int S, bool BONDS = true>
-__device__ __forceinline__ StripThread strip_thread(const StripArgs &a) {
+template <int BX, int S>
+__device__ __forceinline__ StripThread<BX> strip_thread(const StripArgs &a) {
     const StripGeom &g = a.g;
-    StripThread p;
+    StripThread<BX> p;
     const int t = threadIdx.x;
-    p.slot = t / g.nt;                           // column of the workgroup this thread works on
+    p.slot = t / g.nthr;                         // column of the workgroup this thread works on
     p.act = p.slot < g.cols;
-    p.tl = p.act ? t - p.slot * g.nt : 0;        // idle threads mirror thread 0 (no writes)
-    const int sl = p.act ? p.slot : 0;
-    p.x = p.tl % g.lx;
-    const int k = p.tl / g.lx;
+    const int th = p.act ? t - p.slot * g.nthr : 0;        // idle threads mirror thread 0 (no writes)
+    const int rb = p.act ? p.slot * g.region : 0;
+    const int nbx = (g.lx + BX - 1) / BX;
+    const int k = th / nbx, bx = th - k * nbx;
+    p.x0 = min(bx * BX, g.lx - BX);
+    p.skx = bx * BX - p.x0;
     p.y0 = min(k * S, g.ly - S);
-    p.skip = k * S - p.y0;                       // sites shared with the previous strip
-    const int rb = sl * g.region;
-    const int zero = rb + g.lx * g.lyp;          // holds 0: the absent neighbour of an open edge
-    p.base = rb + p.x * g.lyp + p.y0;
-    // neighbour strips (x +- 1) and the strip ends' outside neighbours
-    // (y0 - 1, y0 + S); an absent x neighbour reads the own strip (its bond
-    // value is 0), an absent y neighbour the zero entry
-    p.xp = p.x + 1 < g.lx ? p.base + g.lyp : (g.px ? rb + p.y0 : p.base);
-    p.xm = p.x > 0 ? p.base - g.lyp : (g.px ? rb + (g.lx - 1) * g.lyp + p.y0 : p.base);
-    p.lo = p.y0 > 0 ? p.base - 1 : (g.py ? rb + p.x * g.lyp + g.ly - 1 : zero);
-    p.hi = p.y0 + S < g.ly ? p.base + S : (g.py ? rb + p.x * g.lyp : zero);
-    if constexpr (BONDS) {
-        const double2 *sv = a.poly[0].stval;
-        p.hyp = sv[p.tl];
-        p.hym = sv[g.nt + p.tl];
-        p.hxp = sv[2 * g.nt + p.tl];
-        p.hxm = sv[3 * g.nt + p.tl];
-    }
+    p.sky = k * S - p.y0;
+    p.tl = k * g.lx + p.x0;                      // the block's first strip
+    p.zero = rb + g.region - 1;
+#pragma unroll
+    for (int i = 0; i < BX; ++i) p.cb[i] = rb + strip_run(g, p.x0 + i) + p.y0;
+    // an absent x neighbour reads the own column (its bond value is 0), an
+    // absent y neighbour the zero entry
+    const int xr = p.x0 + BX < g.lx ? p.x0 + BX : (g.px ? 0 : g.lx - 1);
+    const int xl = p.x0 > 0 ? p.x0 - 1 : (g.px ? g.lx - 1 : 0);
+    p.xr = rb + strip_run(g, xr) + p.y0;
+    p.xl = rb + strip_run(g, xl) + p.y0;
+    p.lo = p.y0 > 0 ? -1 : (g.py ? g.ly - 1 : kNoSite);
+    p.hi = p.y0 + S < g.ly ? S : (g.py ? S - g.ly : kNoSite);
     return p;
+}
+
+// a block's bond values: y + 1 of each column (y - 1: its conjugate), and the
+// x bonds between its columns and to the left and right of it, each as the
+// value that multiplies the site to the right of it (for the site to the left:
+// its conjugate)
+template <int BX>
+struct StripBonds {
+    double2 hy[BX], hx[BX + 1];
+};
+template <int BX, bool XR>
+__device__ __forceinline__ StripBonds<BX> strip_bonds(const double2 *stval, int nt, int tl) {
+    ConstGlobalVec2 *sv = (ConstGlobalVec2 *)stval;
+    StripBonds<BX> b;
+#pragma unroll
+    for (int i = 0; i < BX; ++i) {
+        const vec2 u = sv[tl + i], h = sv[2 * nt + tl + i];
+        b.hy[i] = make_double2(u.x, u.y);
+        b.hx[i + 1] = make_double2(h.x, XR ? 0.0 : h.y);
+    }
+    const vec2 h = sv[3 * nt + tl];
+    b.hx[0] = make_double2(h.x, XR ? 0.0 : -h.y);
+    return b;
 }
 
 // One column group of a strip pass, its columns already in LDS (with the
 // zero slot set).  TOUT: the result is written conjugate-transposed
 // (Y[s, j] = conj(y_s)), else plainly; XR: the x bonds are real (Landau
 // gauge, no field).  TWO: a.npoly polynomials in turn, each with its bond
-// values loaded when it starts (else one, its bond values in p).  At the end
+// values loaded when it starts (else one, its bond values in p1).  At the end
 // the next group (na, njb, when next) is loaded into LDS with its zero slot,
 // ready for the next call.
-template <int S, bool TOUT, bool XR, bool TWO>
-__device__ __forceinline__ void strip_group(const StripArgs &a, const StripThread &p, double2 *lds, int64_t jb,
-                                            const StripArgs &na, int64_t njb, bool next) {
+// PHASES: a term in two phases, which needs S to divide ly (rows shared by two
+// blocks would belong to different phases); else in one, its input published
+// before it.
+template <int BX, int S, bool TOUT, bool XR, bool TWO, bool PHASES>
+__device__ __forceinline__ void strip_group(const StripArgs &a, const StripThread<BX> &p, const StripBonds<BX> &p1,
+                                            double2 *lds, int64_t jb, const StripArgs &na, int64_t njb, bool next) {
     const StripGeom &g = a.g;
     const int t = threadIdx.x;
-    const int slot = p.slot, tl = p.tl, x = p.x, y0 = p.y0, skip = p.skip, base = p.base;
-    const int xp = p.xp, xm = p.xm, lo = p.lo, hi = p.hi;
     const bool act = p.act;
     const int wave = t >> 6, lane = t & 63;
-    const int64_t j = jb + slot;
-    double2 xr[S], yv[S];
+    const int64_t j = jb + p.slot;
+    double2 xr[S][BX], yv[S][BX];
 #pragma unroll
-    for (int m = 0; m < S; ++m) {
-        xr[m] = lds[base + m];
-        yv[m] = xr[m];
-    }
+    for (int m = 0; m < S; ++m)
+#pragma unroll
+        for (int i = 0; i < BX; ++i) {
+            xr[m][i] = lds[p.cb[i] + m];
+            yv[m][i] = xr[m][i];
+        }
     for (int ph = 0; ph < (TWO ? a.npoly : 1); ++ph) {
     // this polynomial's parameters (selected, not indexed: a dynamic index
     // into the argument block would copy it to scratch memory)
@@ -237,89 +302,153 @@ __device__ __forceinline__ void strip_group(const StripArgs &a, const StripThrea
     const int PK = pcf ? cf->K : (ph ? a.poly[1].K : a.poly[0].K);
     const int preps = pcf ? cf->reps : (ph ? a.poly[1].reps : a.poly[0].reps);
     const double pdts = ph ? a.poly[1].dts : a.poly[0].dts;
-    double2 hyp = p.hyp, hym = p.hym, hxp = p.hxp, hxm = p.hxm;
+    StripBonds<BX> b = p1;
     if constexpr (TWO) {
-        // bond values (x bonds: real parts only when XR); the opaque copy
-        // keeps their four addresses from being hoisted out of the loops
-        int tq = tl;
+        // the opaque copy keeps the addresses from being hoisted out of the
+        // loops
+        int tq = p.tl;
         asm volatile("" : "+v"(tq));
-        hyp = stv[tq];
-        hym = stv[g.nt + tq];
-        hxp = XR ? make_double2(stv[2 * g.nt + tq].x, 0.0) : stv[2 * g.nt + tq];
-        hxm = XR ? make_double2(stv[3 * g.nt + tq].x, 0.0) : stv[3 * g.nt + tq];
+        b = strip_bonds<BX, XR>(stv, g.nt, tq);
     }
-    // One Horner term: publish the input (unless the column just loaded is
-    // it), then every site of the strip in turn, upwards (UP) or downwards.
-    // A site's new value takes the register its neighbour's old value leaves
-    // free, one place over in the sweep's direction; alternating the
-    // direction puts the values back in place after two terms instead of
-    // moving them all at the loop's end.  Each site's arithmetic is the same
-    // either way.
-    auto term = [&](int kk, bool publish, auto up) {
-        constexpr bool UP = decltype(up)::value;
-        if (publish) {
-            // the previous term's reads are done; publish this term's input
-            __syncthreads();
-            if (act) {
+    // a small block keeps its diagonal in registers, a large one streams it
+    // from L2 a row ahead
+    constexpr bool DREG = BX * S <= 12;
+    double dr[DREG ? S : 1][BX];
+    if constexpr (DREG) {
 #pragma unroll
-                for (int m = 0; m < S; ++m) lds[base + m] = yv[m];
-            }
-            __syncthreads();
-        }
+        for (int m = 0; m < S; ++m)
+#pragma unroll
+            for (int i = 0; i < BX; ++i) dr[m][i] = ((ConstGlobalDouble *)sdg)[m * g.nt + p.tl + i];
+    }
+    // One Horner term in two phases of rows: the edge rows (E first and E
+    // last ones), then the middle ones.  While a phase computes, the other's
+    // rows go to LDS, where a neighbour reads them: the middle rows of the
+    // term before during the edge phase, the new edge rows during the middle
+    // one.  Every value read in a phase was written a barrier ago and is
+    // overwritten a barrier later, so the writes (as dear as three reads)
+    // cost no phase of their own, and one LDS copy does.
+    // UP: the rows of each segment upwards, else downwards.  A site's new
+    // value takes the register its neighbour's old value leaves free, one row
+    // over in the sweep's direction; alternating the direction puts the
+    // values back in place after two terms instead of moving them all at the
+    // loop's end.  Each site's arithmetic is the same either way.
+    auto term = [&](int kk, bool publish_first, auto up) {
+        constexpr bool UP = decltype(up)::value;
+        constexpr int E = S / 4 > 0 ? S / 4 : 1, NE = 2 * E, NM = S - NE, NM_ = NM > 0 ? NM : 1;
+        constexpr auto row = [](int r) {
+            const int u = !PHASES || r < E ? r : (r < NE ? S - NE + r : r - E);
+            return UP ? u : S - 1 - u;
+        };
+        // (an idle thread holds and writes what thread 0 does)
+        auto publish = [&](int m) {
+#pragma unroll
+            for (int i = 0; i < BX; ++i)
+                if (m == 0 || m == S - 1 || i == 0 || i == BX - 1)
+                    lds[p.cb[i] + m] = yv[m][i];
+        };
         const double c = pcf ? cf->ck[kk]
                              : (kk <= kStripMaxK ? (ph ? a.poly[1].ck[kk] : a.poly[0].ck[kk]) : pdts / (double)kk);
-        // opaque copy: keeps the S diagonal addresses from being hoisted
-        // out of the term loop into registers
+        // opaque copy: keeps the diagonal addresses from being hoisted out of
+        // the term loop into registers
         int ntq = g.nt;
         asm volatile("" : "+s"(ntq));
-        const double *sd = sdg + tl;
-        // the old value behind the sweep (first: the strip's outside
-        // neighbour where the sweep starts) and the one past its end
-        double2 back = lds[UP ? lo : hi];
-        const double2 endv = lds[UP ? hi : lo];
+        ConstGlobalDouble *sd = (ConstGlobalDouble *)sdg + p.tl;
+        constexpr int kAhead = BX == 1 ? 4 : (BX == 2 && S <= 8 ? 3 : (PHASES ? 1 : 2));
+        double dv[S][BX];
+#pragma unroll
+        for (int r = 0; r < (DREG ? S : kAhead); ++r)
+#pragma unroll
+            for (int i = 0; i < BX; ++i) dv[row(r)][i] = DREG ? dr[row(r)][i] : sd[row(r) * ntq + i];
+        if (!PHASES && publish_first) {
+            // the previous term's reads are done; publish this term's input
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < S; ++m) publish(m);
+            __syncthreads();
+        }
+        // the sites outside the block, below and above
+        auto outside = [&](bool above, int i) {
+            const int o = above ? p.hi : p.lo;
+            return lds[o == kNoSite ? p.zero : p.cb[i] + o];
+        };
+        double2 back[BX], keep[2][BX], endv[BX];         // keep: the old edge rows next to the middle ones, by segment
         double2 av[S], bv[S];
-        double dv[S];
 #pragma unroll
-        for (int i = 0; i < kLdsAhead && i < S; ++i) {
-            const int m = UP ? i : S - 1 - i;
-            av[m] = lds[xp + m];
-            bv[m] = lds[xm + m];
-        }
+        for (int i = 0; i < BX; ++i) back[i] = outside(!UP, i);
 #pragma unroll
-        for (int i = 0; i < kDiagAhead && i < S; ++i) {
-            const int m = UP ? i : S - 1 - i;
-            dv[m] = sd[m * ntq];
-        }
-#pragma unroll
-        for (int i = 0; i < S; ++i) {
-            const int m = UP ? i : S - 1 - i;
-            if (i + kLdsAhead < S) {
-                const int mf = UP ? m + kLdsAhead : m - kLdsAhead;
-                av[mf] = lds[xp + mf];
-                bv[mf] = lds[xm + mf];
+        for (int r = 0; r < S; ++r) {
+            const int m = row(r);
+            if (r == 0 || (PHASES && r == NE)) {
+                av[m] = lds[p.xl + m];
+                bv[m] = lds[p.xr + m];
             }
-            if (i + kDiagAhead < S) {
-                const int mf = UP ? m + kDiagAhead : m - kDiagAhead;
-                dv[mf] = sd[mf * ntq];
+            // a segment's first row: the old row behind it
+            if (PHASES && r == E) {
+#pragma unroll
+                for (int i = 0; i < BX; ++i) {
+                    back[i] = NM > 0 ? yv[UP ? S - E - 1 : E][i] : keep[0][i];
+                }
             }
-            const double2 ahead = i + 1 < S ? yv[UP ? m + 1 : m - 1] : endv;
-            const double2 cur = yv[m];
-            const double2 nyp = UP ? ahead : back;     // site y + 1 (old value)
-            const double2 nym = UP ? back : ahead;     // site y - 1 (old value)
-            double2 acc = make_double2(dv[m] * cur.x, dv[m] * cur.y);
-            cmac(acc, hyp, nyp);
-            cmac(acc, hym, nym);
-            hmac<XR>(acc, hxp, av[m]);
-            hmac<XR>(acc, hxm, bv[m]);
-            back = cur;
-            // y_new = x + (-i c) acc
-            yv[m] = make_double2(fma(c, acc.y, xr[m].x), fma(-c, acc.x, xr[m].y));
-            // one site at a time: bounds the live neighbour values
-            __builtin_amdgcn_sched_barrier(0);
+            if (r == (PHASES ? (E > 2 ? NE - 2 : NE - 1) : (BX > 1 ? S - 1 : S - 2))) {
+#pragma unroll
+                for (int i = 0; i < BX; ++i) endv[i] = outside(UP, i);
+            }
+            if (PHASES && r == NE) {
+#pragma unroll
+                for (int i = 0; i < BX; ++i) back[i] = keep[0][i];
+            }
+            if (r + 1 < (PHASES && r < NE ? NE : S)) {
+                av[row(r + 1)] = lds[p.xl + row(r + 1)];
+                bv[row(r + 1)] = lds[p.xr + row(r + 1)];
+            }
+            double2 left = av[m];
+#pragma unroll
+            for (int i = 0; i < BX; ++i) {
+                if (!DREG && r + kAhead < S) dv[row(r + kAhead < S ? r + kAhead : r)][i] = sd[row(r + kAhead < S ? r + kAhead : r) * ntq + i];
+                const double2 cur = yv[m][i];
+                const int mn = UP ? m + 1 : m - 1;           // the row ahead
+                const double2 ahead = r == (PHASES ? NE : S) - 1 ? endv[i]
+                                      : PHASES && r == S - 1     ? keep[1][i]
+                                                                 : yv[mn < 0 ? 0 : (mn < S ? mn : S - 1)][i];
+                if (PHASES && r == E - 1) keep[0][i] = cur;
+                if (PHASES && r == E) keep[1][i] = cur;
+                const double2 nyp = UP ? ahead : back[i];     // site y + 1 (old value)
+                const double2 nym = UP ? back[i] : ahead;     // site y - 1 (old value)
+                const double2 right = i + 1 < BX ? yv[m][i + 1] : bv[m];
+                double2 acc = make_double2(dv[m][i] * cur.x, dv[m][i] * cur.y);
+                cmac(acc, b.hy[i], nyp);
+                cmac(acc, make_double2(b.hy[i].x, -b.hy[i].y), nym);
+                hmac<XR>(acc, b.hx[i + 1], right);
+                hmac<XR>(acc, make_double2(b.hx[i].x, -b.hx[i].y), left);
+                back[i] = cur;
+                left = cur;
+                // y_new = x + (-i c) acc
+                yv[m][i] = make_double2(fma(c, acc.y, xr[m][i].x), fma(-c, acc.x, xr[m][i].y));
+                // (opaque: the sum stays in this phase instead of moving, with
+                // its operands, to where the value is next used)
+                asm volatile("" : "+v"(yv[m][i].x), "+v"(yv[m][i].y));
+                if (PHASES && i == 0) {
+                    // the other phase's rows, a row's share at a time
+                    if (r < NE) {
+#pragma unroll
+                        for (int q = r * NM / NE; q < (r + 1) * NM / NE; ++q) publish(E + q);
+                    } else {
+#pragma unroll
+                        for (int q = (r - NE) * NE / NM_; q < (r - NE + 1) * NE / NM_; ++q) publish(row(q));
+                    }
+                }
+                // one site at a time: bounds the live neighbour values
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (PHASES && (r == NE - 1 || r == S - 1)) __syncthreads();
+        }
+        if (PHASES && NM == 0) {
+#pragma unroll
+            for (int m = 0; m < S; ++m) publish(m);
+            __syncthreads();
         }
     };
     for (int rr = 0; rr < preps; ++rr) {
-        // (the first term reads the loaded column from LDS)
         int kk = PK;
         for (; kk >= 2; kk -= 2) {
             term(kk, ph > 0 || rr > 0 || kk != PK, std::true_type{});
@@ -331,12 +460,14 @@ __device__ __forceinline__ void strip_group(const StripArgs &a, const StripThrea
         // the next repetition (or polynomial) acts on this one's result
         if (rr + 1 < preps || (TWO && ph + 1 < a.npoly)) {
 #pragma unroll
-            for (int m = 0; m < S; ++m) xr[m] = yv[m];
+            for (int m = 0; m < S; ++m)
+#pragma unroll
+                for (int i = 0; i < BX; ++i) xr[m][i] = yv[m][i];
         }
     }
     }
     // the last term's LDS reads are done
-    __syncthreads();
+    if (!PHASES) __syncthreads();
     if constexpr (TOUT) {
         // the next column group loads while this one's results leave from
         // registers: Y[s, j] = conj(y_s), a column of the result is a row of Y
@@ -344,11 +475,14 @@ __device__ __forceinline__ void strip_group(const StripArgs &a, const StripThrea
         if (act && j < a.ncols) {
             int64_t ldq = a.ld;
             asm volatile("" : "+s"(ldq));
-            double2 *yo = a.Y + ((int64_t)x * g.ly + y0) * ldq + j;
 #pragma unroll
-            for (int m = 0; m < S; ++m) {
-                if (m >= skip) *yo = make_double2(yv[m].x, -yv[m].y);
-                yo += ldq;
+            for (int i = 0; i < BX; ++i) {
+                GlobalVec2 *yo = (GlobalVec2 *)a.Y + ((int64_t)(p.x0 + i) * g.ly + p.y0) * ldq + j;
+#pragma unroll
+                for (int m = 0; m < S; ++m) {
+                    if (i >= p.skx && m >= p.sky) *yo = vec2{yv[m][i].x, -yv[m][i].y};
+                    yo += ldq;
+                }
             }
         }
     } else {
@@ -357,7 +491,9 @@ __device__ __forceinline__ void strip_group(const StripArgs &a, const StripThrea
         // one request each); then the next group loads
         if (act) {
 #pragma unroll
-            for (int m = 0; m < S; ++m) lds[base + m] = yv[m];
+            for (int m = 0; m < S; ++m)
+#pragma unroll
+                for (int i = 0; i < BX; ++i) lds[p.cb[i] + m] = yv[m][i];
         }
         __syncthreads();
         strip_store(a, lds, jb, wave, lane);
@@ -367,11 +503,11 @@ __device__ __forceinline__ void strip_group(const StripArgs &a, const StripThrea
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // the next group's zero slots (past its sites: the loads leave them alone)
-    if (next && t < na.g.cols) lds[t * na.g.region + na.g.lx * na.g.lyp] = make_double2(0.0, 0.0);
+    if (next && t < na.g.cols) lds[(t + 1) * na.g.region - 1] = make_double2(0.0, 0.0);
     __syncthreads();
 }
 
-template <int S, bool TOUT, bool XR, bool TWO>
+template <int BX, int S, bool TOUT, bool XR, bool TWO, bool PHASES>
 __global__ void __launch_bounds__(kStripThreads) strip_kernel(StripArgs a) {
     extern __shared__ double2 lds[];
     // a polynomial the host did not see: nothing to do unless it is the one
@@ -389,14 +525,16 @@ __global__ void __launch_bounds__(kStripThreads) strip_kernel(StripArgs a) {
         const int64_t t0 = (int64_t)clock64();
         while ((int64_t)clock64() - t0 < a.stagger) __builtin_amdgcn_s_sleep(16);
     }
-    if (t < g.cols) lds[t * g.region + g.lx * g.lyp] = make_double2(0.0, 0.0);
+    if (t < g.cols) lds[(t + 1) * g.region - 1] = make_double2(0.0, 0.0);
     if (jb < a.ncols) strip_dma(a, lds, jb, wave, lane);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    const StripThread p = strip_thread<S, !TWO>(a);
+    const StripThread<BX> p = strip_thread<BX, S>(a);
+    StripBonds<BX> b{};
+    if constexpr (!TWO) b = strip_bonds<BX, XR>(a.poly[0].stval, g.nt, p.tl);
     while (jb < a.ncols) {
         const int64_t rn = r + a.nprog, jbn = rn * g.cols;
-        strip_group<S, TOUT, XR, TWO>(a, p, lds, jb, a, jbn, jbn < a.ncols);
+        strip_group<BX, S, TOUT, XR, TWO, PHASES>(a, p, b, lds, jb, a, jbn, jbn < a.ncols);
         r = rn;
         jb = jbn;
     }
@@ -417,11 +555,15 @@ __device__ __forceinline__ int strip_member_of(const int64_t *__restrict__ ustar
 template <bool TOUT, bool XR>
 __device__ __forceinline__ void strip_group_s(const StripArgs &a, double2 *lds, int64_t jb, const StripArgs &na,
                                               int64_t njb, bool next) {
-    switch (a.g.s) {
-#define LMH_STRIP_GROUP(SS) \
-    case SS: strip_group<SS, TOUT, XR, false>(a, strip_thread<SS>(a), lds, jb, na, njb, next); break;
-        LMH_STRIP_GROUP(4) LMH_STRIP_GROUP(6) LMH_STRIP_GROUP(8) LMH_STRIP_GROUP(10) LMH_STRIP_GROUP(12)
-        LMH_STRIP_GROUP(16) LMH_STRIP_GROUP(18) LMH_STRIP_GROUP(20)
+    switch (strip_shape_id(a.g.bx, a.g.s)) {
+#define LMH_STRIP_GROUP(BX, S)                                                                             \
+    case strip_shape_id(BX, S): {                                                                          \
+        const StripThread<BX> p = strip_thread<BX, S>(a);                                                  \
+        const StripBonds<BX> b = strip_bonds<BX, XR>(a.poly[0].stval, a.g.nt, p.tl);                       \
+        strip_group<BX, S, TOUT, XR, false, false>(a, p, b, lds, jb, na, njb, next);                       \
+        break;                                                                                             \
+    }
+        LMH_STRIP_SHAPES(LMH_STRIP_GROUP)
 #undef LMH_STRIP_GROUP
         default: break;
     }
@@ -442,7 +584,7 @@ __global__ void __launch_bounds__(kStripThreads) batched_strip_kernel(const Stri
     if (u >= nunits) return;
     int m = strip_member_of(ustart, nm, u);
     int64_t jb = (u - ustart[m]) * members[m].g.cols;
-    if (t < members[m].g.cols) lds[t * members[m].g.region + members[m].g.lx * members[m].g.lyp] = make_double2(0.0, 0.0);
+    if (t < members[m].g.cols) lds[(t + 1) * members[m].g.region - 1] = make_double2(0.0, 0.0);
     strip_dma(members[m], lds, jb, wave, lane);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -476,56 +618,52 @@ __global__ void __launch_bounds__(256) strip_snapshot_kernel(const double2 *__re
     if (blockIdx.x == 0 && threadIdx.x == 0) *coef_out = *coef;
 }
 
-template <int S, bool T, bool XR, bool TWO>
-const void *strip_fn() {
-    return (const void *)strip_kernel<S, T, XR, TWO>;
-}
-
 // the dynamic-LDS attribute, once per device and instantiation
-template <int S, bool T, bool XR, bool TWO = false>
+template <int BX, int S, bool T, bool XR, bool TWO, bool PHASES>
 hipError_t strip_attr() {
     static std::atomic<uint64_t> done{0};
     return once_per_device(done, [] {
-        return hipFuncSetAttribute(strip_fn<S, T, XR, TWO>(), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   kStripLdsBytes);
+        return hipFuncSetAttribute((const void *)strip_kernel<BX, S, T, XR, TWO, PHASES>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, kStripLdsBytes);
     });
 }
 
-template <int S, bool T, bool XR, bool TWO>
+template <int BX, int S, bool T, bool XR, bool TWO, bool PHASES>
 hipError_t launch_s(const StripArgs &a, size_t lds, hipStream_t st) {
-    hipError_t e = strip_attr<S, T, XR, TWO>();
+    hipError_t e = strip_attr<BX, S, T, XR, TWO, PHASES>();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((strip_kernel<S, T, XR, TWO>), dim3((unsigned)a.nprog), dim3(kStripThreads), lds, st, a);
+    hipLaunchKernelGGL((strip_kernel<BX, S, T, XR, TWO, PHASES>), dim3((unsigned)a.nprog), dim3((unsigned)a.g.threads), lds,
+                       st, a);
     return hipGetLastError();
 }
 
 // two polynomials in one launch only with conjugate-transposed stores
-template <int S>
+template <int BX, int S, bool PHASES>
 hipError_t launch_sx(bool tout, bool xr, const StripArgs &a, size_t lds, hipStream_t st) {
     if (a.npoly > 1)
-        return xr ? launch_s<S, true, true, true>(a, lds, st) : launch_s<S, true, false, true>(a, lds, st);
-    if (tout) return xr ? launch_s<S, true, true, false>(a, lds, st) : launch_s<S, true, false, false>(a, lds, st);
-    return xr ? launch_s<S, false, true, false>(a, lds, st) : launch_s<S, false, false, false>(a, lds, st);
+        return xr ? launch_s<BX, S, true, true, true, PHASES>(a, lds, st) : launch_s<BX, S, true, false, true, PHASES>(a, lds, st);
+    if (tout)
+        return xr ? launch_s<BX, S, true, true, false, PHASES>(a, lds, st) : launch_s<BX, S, true, false, false, PHASES>(a, lds, st);
+    return xr ? launch_s<BX, S, false, true, false, PHASES>(a, lds, st) : launch_s<BX, S, false, false, false, PHASES>(a, lds, st);
 }
 
-template <int S>
+template <int BX, int S, bool PHASES>
 hipError_t prepare_sx() {
-    hipError_t e = strip_attr<S, true, true>();
-    if (e == hipSuccess) e = strip_attr<S, true, false>();
-    if (e == hipSuccess) e = strip_attr<S, false, true>();
-    if (e == hipSuccess) e = strip_attr<S, false, false>();
-    if (e == hipSuccess) e = strip_attr<S, true, true, true>();
-    if (e == hipSuccess) e = strip_attr<S, true, false, true>();
+    hipError_t e = strip_attr<BX, S, true, true, false, PHASES>();
+    if (e == hipSuccess) e = strip_attr<BX, S, true, false, false, PHASES>();
+    if (e == hipSuccess) e = strip_attr<BX, S, false, true, false, PHASES>();
+    if (e == hipSuccess) e = strip_attr<BX, S, false, false, false, PHASES>();
+    if (e == hipSuccess) e = strip_attr<BX, S, true, true, true, PHASES>();
+    if (e == hipSuccess) e = strip_attr<BX, S, true, false, true, PHASES>();
     return e;
 }
 
-#define LMH_STRIP_LENGTHS(X) X(4) X(6) X(8) X(10) X(12) X(16) X(18) X(20)
-
-hipError_t dispatch_s(int s, bool tout, bool xr, const StripArgs &a, size_t lds, hipStream_t st) {
-    switch (s) {
-#define LMH_STRIP_CASE(S) \
-    case S: return launch_sx<S>(tout, xr, a, lds, st);
-        LMH_STRIP_LENGTHS(LMH_STRIP_CASE)
+hipError_t dispatch_s(bool tout, bool xr, const StripArgs &a, size_t lds, hipStream_t st) {
+    switch (strip_shape_id(a.g.bx, a.g.s)) {
+#define LMH_STRIP_CASE(BX, S) \
+    case strip_shape_id(BX, S):                                                                       \
+        return a.g.ly % S ? launch_sx<BX, S, strip_whole(BX, S)>(tout, xr, a, lds, st) : launch_sx<BX, S, true>(tout, xr, a, lds, st);
+        LMH_STRIP_SHAPES(LMH_STRIP_CASE)
 #undef LMH_STRIP_CASE
         default: return hipErrorInvalidValue;
     }
@@ -563,6 +701,52 @@ bool has_entry(const int32_t *col, int64_t n, int zmax, int64_t i, int64_t j) {
     return false;
 }
 
+// The block shape, workgroup size and columns per workgroup of an lx x ly
+// grid: those of least cost, the rounds of workgroups a CU takes (256 CUs of
+// 8 waves) times 25 (the barriers, latencies and launch of a round) plus its
+// waves' sites per thread (a wave takes its SIMD's time whether or not the
+// others have one), times 1.5 for whole strips (42 LDS reads per 20 sites
+// instead of 24), 1.05 for 4 x 4 (a few spills) and 0.97 for 2 x 10 (it fills a
+// batch's workgroups best).  Fitted to a step's launch (K = 8 twice): at
+// 64 x 64 2 x 8 482 us, 4 x 4 515, 2 x 4 550, 2 x 6 592; at 80 x 80 4 x 4 1094,
+// 2 x 8 1114, 2 x 10 1207; at 100 x 100 2 x 10 2252, 1 x 20 2715; at 37 x 23 2 x 4 30,
+// 2 x 8 36, 2 x 6 38; at 24 x 24 2 x 4 24, 2 x 8 30, 2 x 10 35.
+bool strip_shape(int64_t lx, int64_t ly, StripGeom *g) {
+    const int64_t n = lx * ly;
+    double best = 1e300;
+    for (const StripShape &sh : kStripShapes) {
+        if (sh.bx > lx || sh.s > ly) continue;
+        if (strip_whole(sh.bx, sh.s) && (lx % sh.bx || ly % sh.s)) continue;
+        const int64_t nbx = (lx + sh.bx - 1) / sh.bx, q = (ly + sh.s - 1) / sh.s, nthr = nbx * q;
+        const int64_t lyp = (sh.bx * ly) | 1, region = nbx * lyp + 1;
+        for (int64_t threads = (nthr + 63) / 64 * 64; threads <= kStripThreads; threads += 64) {
+            const int64_t cols = std::min<int64_t>(threads / nthr, kStripLdsBytes / (16 * region));
+            if (cols < 1) continue;
+            const int64_t groups = (n + cols - 1) / cols;
+            const int64_t fit = std::min<int64_t>(kStripThreads / threads, kStripLdsBytes / (16 * region * cols));
+            const int64_t per_cu = std::min<int64_t>(fit, (groups + 255) / 256);
+            const int64_t rounds = (groups + 256 * per_cu - 1) / (256 * per_cu);
+            const int64_t waves = (per_cu * (threads / 64) + 3) / 4 * 4;
+            const double cost = (double)rounds * (25.0 + (double)(waves * sh.bx * sh.s)) *
+                                (sh.bx == 1 ? 1.5 : (strip_whole(sh.bx, sh.s) ? 1.05 : (sh.s == 10 ? 0.97 : 1.0)));
+            if (cost >= best) continue;
+            best = cost;
+            g->lx = (int)lx;
+            g->ly = (int)ly;
+            g->lyp = (int)lyp;
+            g->bx = sh.bx;
+            g->s = sh.s;
+            g->q = (int)q;
+            g->nt = (int)(lx * q);
+            g->nthr = (int)nthr;
+            g->threads = (int)threads;
+            g->cols = (int)cols;
+            g->region = (int)region;
+        }
+    }
+    return best < 1e300;
+}
+
 }  // namespace
 
 bool strip_detect(const int32_t *col, int64_t n, int zmax, StripGeom *g, int32_t *sslot) {
@@ -582,42 +766,14 @@ bool strip_detect(const int32_t *col, int64_t n, int zmax, StripGeom *g, int32_t
         const int py = ly >= 3 && has_entry(col, n, zmax, ly - 1, 0);
         const int px = lx >= 3 && has_entry(col, n, zmax, (lx - 1) * ly, 0);
         if (!try_grid(col, n, zmax, lx, ly, px, py, sslot)) continue;
-        // strip length: the least overlap (then the longest strip) that fits
-        // 512 threads and one column's LDS copy
-        const int lyp = (int)(ly | 1);
-        const int64_t region = lx * lyp + 1;
-        const int64_t cols_lds = kStripLdsBytes / (16 * region);
-        if (cols_lds < 1) continue;
-        int best = 0;
-        double best_ratio = 1e300;
-        for (int s : kStripS) {
-            if (s > ly) continue;
-            const int64_t qn = (ly + s - 1) / s, nt = lx * qn;
-            if (nt > kStripThreads) continue;
-            const double ratio = (double)(qn * s) / (double)ly;
-            if (ratio < best_ratio - 1e-12 || (ratio <= best_ratio + 1e-12 && s > best)) {
-                best = s;
-                best_ratio = ratio;
-            }
-        }
-        if (!best) continue;
-        g->lx = (int)lx;
-        g->ly = (int)ly;
-        g->lyp = lyp;
+        if (ly < 4 || !strip_shape(lx, ly, g)) continue;
         g->px = px;
         g->py = py;
-        g->s = best;
-        g->q = (int)((ly + best - 1) / best);
-        g->nt = (int)lx * g->q;
-        g->cols = (int)std::min<int64_t>(kStripThreads / g->nt, cols_lds);
-        g->region = (int)region;
         return true;
     }
     std::fill(sslot, sslot + 4 * n, -1);
     return false;
 }
-
-int64_t strip_thread_count(const StripGeom &g) { return g.nt; }
 
 namespace {
 
@@ -665,16 +821,19 @@ hipError_t launch_args(const DevHam &h, StripArgs &a, int64_t ncols, bool tout, 
     hipError_t e = device_cus(&cus);
     if (e != hipSuccess) return e;
     const int64_t groups = (ncols + g.cols - 1) / g.cols;
-    const int64_t np = std::min<int64_t>(groups, std::max(cus, 1));
+    const size_t lds = (size_t)g.cols * g.region * sizeof(double2);
+    const int64_t per_cu = std::min<int64_t>(kStripThreads / g.threads, kStripLdsBytes / (int64_t)lds);
+    const int64_t np = std::min<int64_t>(groups, per_cu * std::max(cus, 1));
     a.nprog = ((np + kNumXCD - 1) / kNumXCD) * kNumXCD;
     // half a column period in shader cycles (measured at N = 10^4, S = 20:
     // ~310 cycles per site and term, ~3.3 cycles per site for the load and
     // store), when each workgroup has several column groups to do
     int64_t terms = 0;
     for (int q = 0; q < a.npoly; ++q) terms += (int64_t)a.poly[q].K * a.poly[q].reps;
-    a.stagger = groups >= 4 * a.nprog ? (int64_t)((310.0 * terms * g.s + 3.3 * (double)h.n * g.cols) / 2.0) : 0;
-    const size_t lds = (size_t)g.cols * g.region * sizeof(double2);
-    return dispatch_s(g.s, tout, a.xreal != 0, a, lds, st);
+    a.stagger = per_cu == 1 && groups >= 4 * a.nprog
+                    ? (int64_t)((310.0 * terms * g.bx * g.s + 3.3 * (double)h.n * g.cols) / 2.0)
+                    : 0;
+    return dispatch_s(tout, a.xreal != 0, a, lds, st);
 }
 
 bool strip_shape_ok(const DevHam &h, int64_t ncols, bool tout) {
@@ -732,13 +891,18 @@ hipError_t strip_batch_table(const StripMemberDesc *m, int nm, void **d_args, in
     *d_ustart = nullptr;
     std::vector<StripArgs> args(nm);
     std::vector<int64_t> ustart(nm + 1, 0);
+    // one workgroup per CU with as many columns of a member as it has room
+    // for: more bytes in flight than smaller workgroups with a column each
+    // (12 members of 35 x 35 .. 59 x 59: 1.74 ms per launch against 1.85)
     size_t need = 0;
     for (int i = 0; i < nm; ++i) {
         const DevHam &h = *m[i].h;
         if (h.sg.s == 0 || h.n != (int64_t)h.sg.lx * h.sg.ly) return hipErrorInvalidValue;
         args[i] = strip_args(h, m[i].X, m[i].Y, m[i].ld, h.n, m[i].dts, m[i].K, m[i].reps);
-        ustart[i + 1] = ustart[i] + (h.n + h.sg.cols - 1) / h.sg.cols;
-        need = std::max(need, (size_t)h.sg.cols * h.sg.region * sizeof(double2));
+        StripGeom &g = args[i].g;
+        g.cols = std::min(kStripThreads / g.nthr, (int)(kStripLdsBytes / ((size_t)g.region * sizeof(double2))));
+        need = std::max(need, (size_t)g.cols * g.region * sizeof(double2));
+        ustart[i + 1] = ustart[i] + (h.n + g.cols - 1) / g.cols;
     }
     StripArgs *da = nullptr;
     int64_t *du = nullptr;
@@ -787,11 +951,11 @@ hipError_t launch_batched_strip(const void *d_args, const int64_t *d_ustart, int
 }
 
 hipError_t prepare_strip(const DevHam &h) {
-    switch (h.sg.s) {
-        case 0: return hipSuccess;
-#define LMH_STRIP_PREP(S) \
-    case S: return prepare_sx<S>();
-        LMH_STRIP_LENGTHS(LMH_STRIP_PREP)
+    if (h.sg.s == 0) return hipSuccess;
+    switch (strip_shape_id(h.sg.bx, h.sg.s)) {
+#define LMH_STRIP_PREP(BX, S) \
+    case strip_shape_id(BX, S): return h.sg.ly % S ? prepare_sx<BX, S, strip_whole(BX, S)>() : prepare_sx<BX, S, true>();
+        LMH_STRIP_SHAPES(LMH_STRIP_PREP)
 #undef LMH_STRIP_PREP
         default: return hipErrorInvalidValue;
     }
