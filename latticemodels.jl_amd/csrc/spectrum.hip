@@ -53,8 +53,13 @@ __global__ void __launch_bounds__(256) scale_columns_kernel(double2 *__restrict_
 }
 
 // P = W W^H, W: n x m (column-major, ldw), P: n x n (ldp).
-// Workgroup 256 threads = 4 waves computes a 64x64 tile of P; each wave a
-// 32x32 sub-tile as 2x2 MFMA 16x16 blocks.  MFMA f64 16x16x4 lane layout:
+// Workgroup 256 threads = 4 waves computes a 64x64 tile of P on or below the
+// diagonal and stores it and its conjugate transpose; each wave a
+// 32x32 sub-tile as 2x2 MFMA 16x16 blocks.  Bound by the matrix cores (16 MFMA
+// a step of 4 columns and wave, 512 cycles of its SIMD, for four 1 KB loads
+// from L2, which are taken a step ahead): n = m = 2304 2.45 ms with all
+// tiles and the loads in front of their step, 1.48 now; 8 n^2 m / 2 flops take 0.63
+// at the rate of a large product.  MFMA f64 16x16x4 lane layout:
 //   A (16x4): lane l holds A[l % 16][l / 16]
 //   B (4x16): lane l holds B[l / 16][l % 16]
 //   D (16x16): lane l, element r holds D[l / 16 + 4 * r][l % 16]
@@ -69,8 +74,14 @@ __global__ void __launch_bounds__(256) herk_mfma_kernel(const double2 *__restric
                                                         const double *__restrict__ sgn) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int64_t i0 = (int64_t)blockIdx.x * 64 + (wave & 1) * 32;
-    const int64_t j0 = (int64_t)blockIdx.y * 64 + (wave >> 1) * 32;
+    // tile (bi, bj), bi >= bj, from the workgroup's place in the triangle
+    const int64_t id = blockIdx.x;
+    int64_t bi = (int64_t)((sqrt(8.0 * (double)id + 1.0) - 1.0) * 0.5);
+    while (bi * (bi + 1) / 2 > id) --bi;
+    while ((bi + 1) * (bi + 2) / 2 <= id) ++bi;
+    const int64_t bj = id - bi * (bi + 1) / 2;
+    const int64_t i0 = bi * 64 + (wave & 1) * 32;
+    const int64_t j0 = bj * 64 + (wave >> 1) * 32;
     const int r16 = lane & 15;
     const int k4 = lane >> 4;
     v4d acc_re[2][2], acc_im[2][2];
@@ -81,29 +92,51 @@ __global__ void __launch_bounds__(256) herk_mfma_kernel(const double2 *__restric
             acc_re[a][b] = (v4d){0.0, 0.0, 0.0, 0.0};
             acc_im[a][b] = (v4d){0.0, 0.0, 0.0, 0.0};
         }
-    for (int64_t k0 = 0; k0 < m; k0 += 4) {
-        const int64_t k = k0 + k4;
-        double2 av[2], bv[2];
+    // rows beyond n read row n - 1 (their results are not stored), columns
+    // beyond m column m - 1, taken as 0
+    int64_t ia[2], jb[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        ia[t] = min(i0 + 16 * t + r16, n - 1);
+        jb[t] = min(j0 + 16 * t + r16, n - 1);
+    }
+    double2 av[2], bv[2];
+    double sk = 1.0;
+    auto load = [&](int64_t k) {
+        const double2 *w = W + min(k, m - 1) * ldw;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const int64_t ia = i0 + 16 * t + r16;
-            const int64_t jb = j0 + 16 * t + r16;
-            av[t] = (k < m && ia < n) ? W[k * ldw + ia] : make_double2(0.0, 0.0);
-            bv[t] = (k < m && jb < n) ? W[k * ldw + jb] : make_double2(0.0, 0.0);
+            av[t] = w[ia[t]];
+            bv[t] = w[jb[t]];
         }
-        if (sgn && k < m) {
-            const double sk = sgn[k];
-            bv[0] = make_double2(sk * bv[0].x, sk * bv[0].y);
-            bv[1] = make_double2(sk * bv[1].x, sk * bv[1].y);
+        if (sgn) sk = sgn[min(k, m - 1)];
+    };
+    load(k4);
+    for (int64_t k0 = 0; k0 < m; k0 += 4) {
+        const double f = k0 + k4 < m ? sk : 0.0;
+        double ax[2], ay[2], nx[2], bx[2], by[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            ax[t] = av[t].x;
+            ay[t] = av[t].y;
+            nx[t] = -av[t].x;
+            bx[t] = f * bv[t].x;
+            by[t] = f * bv[t].y;
         }
+        load(k0 + 4 + k4);
 #pragma unroll
         for (int a = 0; a < 2; ++a)
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
-                acc_re[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a].x, bv[b].x, acc_re[a][b], 0, 0, 0);
-                acc_re[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a].y, bv[b].y, acc_re[a][b], 0, 0, 0);
-                acc_im[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a].y, bv[b].x, acc_im[a][b], 0, 0, 0);
-                acc_im[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-av[a].x, bv[b].y, acc_im[a][b], 0, 0, 0);
+                acc_re[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ax[a], bx[b], acc_re[a][b], 0, 0, 0);
+                acc_im[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ay[a], bx[b], acc_im[a][b], 0, 0, 0);
+            }
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                acc_re[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ay[a], by[b], acc_re[a][b], 0, 0, 0);
+                acc_im[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(nx[a], by[b], acc_im[a][b], 0, 0, 0);
             }
     }
 #pragma unroll
@@ -114,7 +147,10 @@ __global__ void __launch_bounds__(256) herk_mfma_kernel(const double2 *__restric
             for (int r = 0; r < 4; ++r) {
                 const int64_t row = i0 + 16 * a + k4 + 4 * r;
                 const int64_t col = j0 + 16 * b + r16;
-                if (row < n && col < n) P[col * ldp + row] = make_double2(acc_re[a][b][r], acc_im[a][b][r]);
+                if (row < n && col < n && row >= col) {
+                    P[col * ldp + row] = make_double2(acc_re[a][b][r], acc_im[a][b][r]);
+                    if (row > col) P[row * ldp + col] = make_double2(acc_re[a][b][r], -acc_im[a][b][r]);
+                }
             }
 }
 
@@ -229,8 +265,10 @@ hipError_t launch_scale_columns(double2 *V, int64_t lda, int64_t n, const double
 
 hipError_t launch_herk(const double2 *W, int64_t ldw, int64_t n, int64_t m, double2 *P, int64_t ldp, hipStream_t st,
                        const double *sgn) {
-    const int64_t nb = (n + 63) / 64;
-    hipLaunchKernelGGL(herk_mfma_kernel, dim3((unsigned)nb, (unsigned)nb), dim3(256), 0, st, W, ldw, n, m, P, ldp, sgn);
+    const int64_t nb = (n + 63) / 64, tiles = nb * (nb + 1) / 2;
+    if (n == 0) return hipSuccess;
+    if (m == 0) return launch_zero(P, ldp * n, st);      // (no column: P = 0)
+    hipLaunchKernelGGL(herk_mfma_kernel, dim3((unsigned)tiles), dim3(256), 0, st, W, ldw, n, m, P, ldp, sgn);
     return hipGetLastError();
 }
 
