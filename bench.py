@@ -51,7 +51,7 @@ LDS_PEAK_TBS = 128 * 256 * 2.4e9 / 1e12  # 128 B/clk per CU, 256 CUs, 2.4 GHz
 #     traffic_bytes_per_launch: <variant> <bytes>
 # `roofline.traffic` is that figure for the variant that ran, with the file
 # it came from; null when no summary covers the variant.
-TRAFFIC_FILES = ("strip_fused_steps_n10000.md", "strip_kernel_n10000.md", "fused_value_classes_n10000.md",
+TRAFFIC_FILES = ("strip_blocks_n10000.md", "strip_fused_steps_n10000.md", "strip_kernel_n10000.md", "fused_value_classes_n10000.md",
                  "fused_column_pass_n10000.md")
 # H bytes each fused variant with one column per workgroup reads from L2 per
 # site and Horner term (zmax <= 4 layouts): the packed record (diagonal +
@@ -848,17 +848,18 @@ def main():
     # Per site and term: the diagonal product (2 multiplies), the two y bonds
     # (4 complex FMAs each), the two x bonds (real when the Landau gauge
     # keeps them real: 2 FMAs each) and the Horner update (2 FMAs) = 30
-    # FLOP; LDS: one 16-byte write and two 16-byte reads
+    # FLOP; LDS: a block of 2 x 10 sites writes its 20 and reads 24 around
+    # it, 16 bytes each
     on_chip = None
     if dom == "fused_left" and variant == _lib.FUSED_STRIP:
         site_terms = terms_per_launch * N * N
         flops = 30.0 * site_terms
-        lds_b = 48.0 * site_terms
+        lds_b = 35.2 * site_terms
         t = avg_ms * 1e-3
         on_chip = {"fp64_TFLOPs": flops / t / 1e12, "fp64_peak_TFLOPs": FP64_PEAK_TFLOPS,
                    "fp64_frac": flops / t / 1e12 / FP64_PEAK_TFLOPS,
                    "lds_TBs": lds_b / t / 1e12, "lds_peak_TBs": LDS_PEAK_TBS, "lds_frac": lds_b / t / 1e12 / LDS_PEAK_TBS,
-                   "accounting": "30 FLOP and 48 B of LDS traffic per site and Horner term (real x bonds); "
+                   "accounting": "30 FLOP and 35.2 B of LDS traffic per site and Horner term (real x bonds); "
                                  "LDS peak 128 B/clk/CU x 256 CUs x 2.4 GHz"}
     # the whole step against the lower of the two floors a fused step has:
     # moving P through HBM twice (read P, write W, read W, write P': 64 N^2 B)
