@@ -466,8 +466,9 @@ __device__ __forceinline__ void strip_group(const StripArgs &a, const StripThrea
         }
     }
     }
-    // the last term's LDS reads are done
-    if (!PHASES) __syncthreads();
+    // the last term's LDS reads are done (or the column's own, when there is
+    // no term)
+    __syncthreads();
     if constexpr (TOUT) {
         // the next column group loads while this one's results leave from
         // registers: Y[s, j] = conj(y_s), a column of the result is a row of Y
