@@ -476,7 +476,8 @@ int lmh_set_step_mode(lmh_context *ctx, int mode);
  *   LMH_OPT_LEFT_PASS   per-term left pass (and the adjoint's reverse terms):
  *                       0 = 3 where it applies, else banded when every entry
  *                       of H lies within 1024 (reverse terms: 512) rows of the
- *                       diagonal, else gather (default), 1 = gather through L1/L2, 2 = banded (a
+ *                       diagonal and no row has more than 12 slots, else gather
+ *                       (default), 1 = gather through L1/L2, 2 = banded (a
  *                       block's rows plus the band staged in LDS per column),
  *                       3 = banded with two Horner terms per launch (band <=
  *                       512 rows; the halo rows' H held in LDS) */

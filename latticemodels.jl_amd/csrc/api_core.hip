@@ -439,8 +439,8 @@ int lmh_set_option(lmh_context *ctx, int key, int64_t value) {
         case LMH_OPT_LEFT_PASS:
             if (value < 0 || value > 3) return fail(LMH_EINVAL, "left-pass variant must be 0 .. 3");
             if (value == 2 && ctx->geom_set && !lmh::left_band_fits(ctx->h))
-                return fail(LMH_ERANGE, "banded left pass needs H's band <= 1024 rows (band = %lld)",
-                            (long long)ctx->h.band);
+                return fail(LMH_ERANGE, "banded left pass needs H's band <= 1024 rows and at most 12 slots per row "
+                            "(band = %lld, zmax = %d)", (long long)ctx->h.band, ctx->h.zmax);
             if (value == 3 && ctx->geom_set && !lmh::left_band2_fits(ctx->h))
                 return fail(LMH_ERANGE, "two-term banded left pass needs H's band <= 512 rows and its halo in LDS "
                             "(band = %lld, zmax = %d)", (long long)ctx->h.band, ctx->h.zmax);

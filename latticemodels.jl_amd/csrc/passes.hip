@@ -382,7 +382,8 @@ int64_t xcd_pad(int64_t nreal) { return ((nreal + kNumXCD - 1) / kNumXCD) * kNum
 
 }  // namespace
 
-bool left_band_fits(const DevHam &h) { return h.band >= 0 && h.band <= kBandRows; }
+// (the banded kernels are compiled for up to 12 slots per row)
+bool left_band_fits(const DevHam &h) { return h.band >= 0 && h.band <= kBandRows && h.zmax <= 12; }
 
 hipError_t launch_horner_left(const DevHam &h, const double2 *X, const double2 *Yin, double2 *Yout, int64_t ld,
                               int64_t ncols, double c, int first, int lcols, hipStream_t st, int variant,
