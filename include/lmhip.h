@@ -474,7 +474,8 @@ int lmh_set_step_mode(lmh_context *ctx, int mode);
  *                       5 = as 1 with each side's result transposed by a
  *                       tiled transpose pass instead of the last term
  *   LMH_OPT_LEFT_PASS   per-term left pass (and the adjoint's reverse terms):
- *                       0 = 3 where it applies, else banded when every entry
+ *                       0 = 3 where it applies and no row has more than 9
+ *                       slots, else banded when every entry
  *                       of H lies within 1024 (reverse terms: 512) rows of the
  *                       diagonal and no row has more than 12 slots, else gather
  *                       (default), 1 = gather through L1/L2, 2 = banded (a

@@ -219,9 +219,13 @@ int step_impl(lmh_context *ctx, lmh_state *st);
 // two terms per launch 11.7 ms) while the right pass sweeps neighbour
 // columns through the caches (18.3 ms per term), so both sides run as left
 // passes with a tiled conjugate transpose (5.0 ms) between them wherever the
-// band fits: a step takes 75 instead of 152 ms at K = 6.
+// band fits: a step takes 75 instead of 152 ms at K = 6.  Two terms per launch
+// only up to 9 slots per row: with 10 .. 12 the rows of both terms exceed the
+// registers (left passes of a step, K = 8, 12 slots: N = 1600 1458 us against
+// 919 for single terms, 4900 7.8 ms / 4.3, 10816 33.8 / 17.5; 9 slots, K = 7:
+// N = 2592 0.79 / 0.95, 7200 6.3 / 7.4, 11250 13.4 / 16.0).
 int step_left(const lmh_context *ctx) {
-    return ctx->left_variant == 0 && lmh::left_band2_fits(ctx->h) ? 3 : ctx->left_variant;
+    return ctx->left_variant == 0 && ctx->h.zmax <= 9 && lmh::left_band2_fits(ctx->h) ? 3 : ctx->left_variant;
 }
 int step_right(const lmh_context *ctx) {
     return !ctx->right_set && lmh::left_band_fits(ctx->h) && ctx->left_variant != 1 ? 5 : ctx->right_variant;
