@@ -87,7 +87,7 @@ int lmh_kets_step(lmh_context *ctx, lmh_kets *k) {
     const int a = k->cur, b = (a + 1) % 3, c = (a + 2) % 3;
     if (lmh::fused_supported(h) && h.n <= ctx->fused_max_n && ctx->step_mode != LMH_STEP_PER_PASS) {
         ProfScope ps(ctx, LMH_KERNEL_FUSED);
-        ctx->fused_launched = lmh::fused_resolved_variant(h, ctx->fused_variant, reps);
+        ctx->fused_launched = lmh::fused_resolved_variant(h, ctx->fused_variant, reps, k->m);
         HIP_TRY(lmh::launch_fused_left(h, k->buf[a], k->buf[b], k->buf[c], k->ld, k->m, ctx->dt / ctx->s, K, reps,
                                        false, ctx->fused_variant, ctx->stream),
                 "fused ket launch");

@@ -406,17 +406,40 @@ bool column_variant_valid(int v, int64_t n, int zmax) {
 // 10.3, 484 10.9 / 14.9, 1024 25 / 33, 1936 74 / 95, 2304 97 / 150, 2916
 // 177 / 222, 3600 288 / 474, 4096 428 / 522); above, H must be streamed and
 // the general kernel's 80 B per site are the smaller stream.  Up to 9 slots
-// (Haldane, K = 6): in registers up to n = 2048 (N = 512 18 / 51, 1984
-// 106 / 146), streamed above (3200 407 / 630, 5000 1005 / 1043, 9800
-// 4547 / 5765).
-int column_default_variant(int64_t n, int zmax) {
+// in registers up to n = 2048 (Haldane, K = 6: N = 512 18 / 51, 1984
+// 106 / 146), streamed above, where the threads' number of rows decides (us
+// per step, K = 7 .. 8, streamed / general): 5 slots N = 2450 361 / 459, 2888
+// 538 / 564, 3528 696 / 1048, 3872 1078 / 1212, 4232 1458 / 1403, 5000 1871 /
+// 1668; 6 slots 2601 520 / 479, 3481 759 / 1047, 3969 1195 / 1238, 4356 1617 /
+// 1428; 8 slots 2500 498 / 530, 2601 668 / 542, 3136 920 / 1115, 3600 1352 /
+// 1318, 4096 1597 / 1407, 5041 2401 / 1911; 9 slots 2450 467 / 613, 2592 644 /
+// 634, 2888 713 / 673, 3528 942 / 1373, 4232 1794 / 1823, 5000 2233 / 2184.
+// So from 6 slots on a sixth row of 512 threads goes to the general kernel
+// (which has 1024 with three each), except that with 9 a wave's worth of it
+// costs nothing; rows past the seventh with 7 or 8 slots, past the eighth with 5 or
+// 6 (with 9 the general kernel loads 12 slots and both are within 2 %).
+// Few columns (at most two to a CU) are one round of either, and the streamed
+// rows the shorter one up to more of them (48 kets: 5 slots N = 3698 50 / 66;
+// 7 slots 3698 69 / 73; 8 slots 2704 55 / 59, 3600 74 / 74, 4096 80 / 75;
+// 9 slots 2592 52 / 70, 4608 84 / 87).
+// Above n = 5120 one column fills the LDS and the streamed rows win again
+// (8 slots 5184 3365 / 5163, 10201 11248 / 11602; 9 slots 10082 10735 / 14073).
+int column_default_variant(int64_t n, int zmax, int64_t ncols) {
     if (zmax <= 4) {
         if (n > 4096) return -1;
         return n <= 128 ? 0 : n <= 256 ? 1 : n <= 512 ? 2 : n <= 1024 ? 4 : n <= 2048 ? 6 : n <= 2304 ? 8
                : n <= 3072 ? 10 : n <= 3840 ? 11 : 12;
     }
     if (zmax > 9 || n > 10240) return -1;
-    return n <= 256 ? 13 : n <= 2048 ? 15 : n <= 2560 ? 16 : n <= 3584 ? 18 : n <= 5120 ? 19 : 20;
+    const bool few = ncols <= 512;
+    if (n <= 2560) return n <= 256 ? 13 : n <= 2048 ? 15 : 16;
+    if (n <= 3072 && zmax > 5 && !few) return zmax == 9 && n <= 2560 + 64 ? 17 : -1;
+    if (n <= 3584) return 18;
+    if (n <= 5120) {
+        const int64_t last = zmax == 9 ? 5120 : zmax == 8 ? 3584 : zmax == 7 ? (few ? 4096 : 3584) : (few ? 5120 : 4096);
+        return n <= last ? 19 : -1;
+    }
+    return 20;
 }
 
 bool column_variant_runs(int v, const DevHam &h, int reps) {

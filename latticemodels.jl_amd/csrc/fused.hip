@@ -489,16 +489,16 @@ bool fused_dict_fits(int v, int64_t n, int ndict) {
 
 int fused_variant_columns(int v) { return v == kStripVariant ? 1 : kVariants[v].c; }
 
-// The kernel above by size (batches, and what the column kernel does not
+int fused_default_variant(int64_t n, int zmax, int64_t ncols) {
+    const int c = column_default_variant(n, zmax, ncols);
+    return c >= 0 ? kColumnVariant0 + c : fused_general_variant(n, zmax);
+}
+
+// This file's kernel by size (batches, and what the column kernel does not
 // take), from timing every variant on square lattices (N = 1024 .. 10^4,
 // K = 8): x held in registers wins at every size; H rows in
 // registers for N <= 1024; above that, for zmax <= 4, the packed site record
 // (diagonal + 16-bit columns, one 16-byte load) beats separate loads by 5-10%.
-int fused_default_variant(int64_t n, int zmax) {
-    const int c = column_default_variant(n, zmax);
-    return c >= 0 ? kColumnVariant0 + c : fused_general_variant(n, zmax);
-}
-
 int fused_general_variant(int64_t n, int zmax) {
     const bool packed = zmax <= 4;
     if (n <= 1024) return packed ? 16 : 19;
@@ -511,9 +511,9 @@ int fused_general_variant(int64_t n, int zmax) {
 // Default variant of a batch size class.
 int fused_batch_variant(int64_t n, int zmax) { return fused_general_variant(n, zmax); }
 
-int fused_resolved_variant(const DevHam &h, int variant, int reps) {
+int fused_resolved_variant(const DevHam &h, int variant, int reps, int64_t ncols) {
     if ((variant < 0 || variant == kStripVariant) && h.strip_ok && h.sg.s > 0) return kStripVariant;
-    int v = variant < 0 || variant == kStripVariant ? fused_default_variant(h.n, h.zmax) : variant;
+    int v = variant < 0 || variant == kStripVariant ? fused_default_variant(h.n, h.zmax, ncols < 0 ? h.n : ncols) : variant;
     if (v >= kColumnVariant0 && !column_variant_runs(v - kColumnVariant0, h, reps)) v = fused_general_variant(h.n, h.zmax);
     if (variant < 0 && fused_default_dict(v) >= 0) v = fused_default_dict(v);
     if (fused_variant_is_dict(v) && !(h.ndict > 0 && h.dict_ok && fused_dict_fits(v, h.n, h.ndict)))
@@ -529,7 +529,7 @@ hipError_t launch_fused_left(const DevHam &h, const double2 *X, double2 *Y, doub
     if ((variant < 0 || variant == kStripVariant) && h.strip_ok && h.sg.s > 0)
         return launch_strip(h, X, Y, ld, ncols, dt_over_s, K, reps, transposed_out, st);
     // (a class table only when the last H build matched it and it fits)
-    const int v = fused_resolved_variant(h, variant, reps);
+    const int v = fused_resolved_variant(h, variant, reps, ncols);
     if (v < kColumnVariant0 && reps > 1 && !scratch) return hipErrorInvalidValue;
     if (!fused_variant_valid(v, h.n, h.zmax)) return hipErrorInvalidValue;
     if (v >= kColumnVariant0)

@@ -349,7 +349,7 @@ int fused_variant_fallback(int v);
 // the class table of ndict entries fits beside the variant's columns in LDS
 bool fused_dict_fits(int v, int64_t n, int ndict);
 int fused_variant_columns(int v);
-int fused_default_variant(int64_t n, int zmax);
+int fused_default_variant(int64_t n, int zmax, int64_t ncols);
 int fused_general_variant(int64_t n, int zmax);
 int fused_batch_variant(int64_t n, int zmax);
 hipError_t prepare_fused(int variant);
@@ -370,14 +370,14 @@ hipError_t launch_conj_transpose(const double2 *A, double2 *B, int64_t n, int64_
 // the variant number of the strip kernel, and the variant a fused launch with
 // `variant` (-1: default) runs for the current H
 int fused_strip_variant();
-int fused_resolved_variant(const DevHam &h, int variant, int reps = 1);
+int fused_resolved_variant(const DevHam &h, int variant, int reps = 1, int64_t ncols = -1);    // ncols: -1 for n
 
 // kernels/launchers (column.hip): fused column pass with H's rows in registers
 // or loaded a site ahead; variants (threads, sites per thread, columns, slots)
 int column_variant_count();
 bool column_variant_valid(int v, int64_t n, int zmax);
 bool column_variant_runs(int v, const DevHam &h, int reps);
-int column_default_variant(int64_t n, int zmax);    // -1: the general kernel
+int column_default_variant(int64_t n, int zmax, int64_t ncols);    // -1: the general kernel
 hipError_t launch_column(int v, const DevHam &h, const double2 *X, double2 *Y, int64_t ld, int64_t ncols,
                          double dt_over_s, int K, int reps, bool tout, hipStream_t st);
 
