@@ -98,7 +98,11 @@ __global__ void __launch_bounds__(kLzThreads) lanczos_beta_kernel(const double *
 // With LDS tree sums (8 barriers each, three sums) and the loads behind the
 // first of them 7.7 us, now 6.1; the kernel below 5.4, now 3.6 (N = 100352,
 // 3 neighbours, one column).
-template <int ZR>
+// AHEAD: H's values and the previous vector are loaded in front of the sum
+// too, which pays while waves are few.  With 9 slots they cost the registers
+// of other waves: 100 kets at N = 20000 69 us a launch with them, 57 without
+// (a step 3.22 and 3.11 ms), one ket 132 and 136 us a step.
+template <int ZR, bool AHEAD>
 __global__ void __launch_bounds__(kLzThreads) lanczos_matvec_kernel(
     const int32_t *__restrict__ col, const double2 *__restrict__ val, const double *__restrict__ diag, int64_t n,
     int zmax, const double2 *__restrict__ W, const double *__restrict__ part_w, double2 *__restrict__ Vj,
@@ -115,23 +119,24 @@ __global__ void __launch_bounds__(kLzThreads) lanczos_matvec_kernel(
 #pragma unroll
     for (int q = 0; q < ZR; ++q) {
         cq[q] = q < zmax ? col[(int64_t)q * n + ic] : -1;
-        if (ZR <= 9 && q < zmax) hv[q] = val[(int64_t)q * n + ic];
+        if (AHEAD && q < zmax) hv[q] = val[(int64_t)q * n + ic];
     }
     double b[1] = {partial_share(part_w + c * nb, nb)};
     const double2 wi = w[ic];
     const double d = diag[ic];
     double2 p = make_double2(0.0, 0.0);
-    if (Vprev) p = Vprev[c * ld + ic];
+    if (AHEAD && Vprev) p = Vprev[c * ld + ic];
     double2 hw = make_double2(d * wi.x, d * wi.y);
 #pragma unroll
     for (int q = 0; q < ZR; ++q)
         if (cq[q] >= 0) {
-            const double2 h = ZR <= 9 ? hv[q] : val[(int64_t)q * n + ic];
+            const double2 h = AHEAD ? hv[q] : val[(int64_t)q * n + ic];
             const double2 x = w[cq[q]];
             hw.x += fma(h.x, x.x, -(h.y * x.y));
             hw.y += fma(h.y, x.x, h.x * x.y);
         }
     block_sums(b, red);
+    if (!AHEAD && Vprev) p = Vprev[c * ld + ic];
     const double beta = sqrt(b[0]);
     const double inv = beta > 0.0 ? 1.0 / beta : 0.0;
     double dot[2] = {0.0, 0.0};                          // conj(v_i) r
@@ -246,15 +251,17 @@ hipError_t launch_lanczos_iteration(const DevHam &h, const double2 *W, const dou
     const int64_t n = h.n;
     const int nb = lanczos_blocks(n);
     const dim3 grid((unsigned)nb, (unsigned)m);
-#define LMH_LZ(ZR)                                                                                                 \
-    hipLaunchKernelGGL(lanczos_matvec_kernel<ZR>, grid, dim3(kLzThreads), 0, st, h.col, h.val, h.diag, n, h.zmax, W, \
-                       part_w, Vj, Vprev, Wn, ld, beta_out, part_re, part_im, nb)
+#define LMH_LZ(ZR, AHEAD)                                                                                          \
+    hipLaunchKernelGGL((lanczos_matvec_kernel<ZR, AHEAD>), grid, dim3(kLzThreads), 0, st, h.col, h.val, h.diag, n,   \
+                       h.zmax, W, part_w, Vj, Vprev, Wn, ld, beta_out, part_re, part_im, nb)
     if (h.zmax <= 4)
-        LMH_LZ(4);
+        LMH_LZ(4, true);
+    else if (h.zmax <= 9 && m <= 8)
+        LMH_LZ(9, true);
     else if (h.zmax <= 9)
-        LMH_LZ(9);
+        LMH_LZ(9, false);
     else if (h.zmax <= 16)
-        LMH_LZ(16);
+        LMH_LZ(16, false);
     else
         return hipErrorInvalidValue;
 #undef LMH_LZ
