@@ -6,6 +6,13 @@
 #include <atomic>
 #include <cstdint>
 
+namespace lmhapi {
+// hipMalloc; when the device is full, the spare buffers on it (api_internal.h)
+// are given back and the allocation is tried once more.  Every device
+// allocation of the library goes through it.
+hipError_t device_malloc(void **p, size_t bytes);
+}  // namespace lmhapi
+
 namespace lmh {
 
 // Runs set() once per device (the current one) for the flag word `done`:

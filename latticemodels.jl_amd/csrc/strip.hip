@@ -907,8 +907,8 @@ hipError_t strip_batch_table(const StripMemberDesc *m, int nm, void **d_args, in
     }
     StripArgs *da = nullptr;
     int64_t *du = nullptr;
-    hipError_t e = hipMalloc((void **)&da, sizeof(StripArgs) * std::max(nm, 1));
-    if (e == hipSuccess) e = hipMalloc((void **)&du, sizeof(int64_t) * (nm + 1));
+    hipError_t e = lmhapi::device_malloc((void **)&da, sizeof(StripArgs) * std::max(nm, 1));
+    if (e == hipSuccess) e = lmhapi::device_malloc((void **)&du, sizeof(int64_t) * (nm + 1));
     if (e == hipSuccess && nm) e = hipMemcpy(da, args.data(), sizeof(StripArgs) * nm, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(du, ustart.data(), sizeof(int64_t) * (nm + 1), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
