@@ -36,17 +36,19 @@ int lmh_kets_create(lmh_context *ctx, int64_t m, lmh_kets **out) {
 
 int lmh_kets_destroy(lmh_kets *k) {
     if (!k) return LMH_OK;
+    lmh_context *keep = nullptr;
     if (k->ctx) {
         (void)hipSetDevice(k->ctx->device);
-        (void)hipDeviceSynchronize();
+        // (a wait that failed, e.g. beside a capture: nothing is kept)
+        if (hipDeviceSynchronize() == hipSuccess) keep = k->ctx;
         k->ctx->kets.erase(k);
     }
-    for (int q = 0; q < 3; ++q) sfree(k->ctx, k->buf[q], (size_t)k->ld * k->m);
+    for (int q = 0; q < 3; ++q) sfree(keep, k->buf[q], (size_t)k->ld * k->m);
     krylov_graphs_free(k);
-    sfree(k->ctx, k->basis, k->basis_cap);
-    sfree(k->ctx, k->lz, k->lz_cap);
-    sfree(k->ctx, k->coef, k->coef_cap);
-    sfree(k->ctx, k->len, k->len_cap);
+    sfree(keep, k->basis, k->basis_cap);
+    sfree(keep, k->lz, k->lz_cap);
+    sfree(keep, k->coef, k->coef_cap);
+    sfree(keep, k->len, k->len_cap);
     if (k->h_pin) (void)hipHostFree(k->h_pin);
     delete k;
     return LMH_OK;

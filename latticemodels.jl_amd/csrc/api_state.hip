@@ -32,20 +32,22 @@ int lmh_state_create(lmh_context *ctx, lmh_state **out) {
 
 int lmh_state_destroy(lmh_state *st) {
     if (!st) return LMH_OK;
+    lmh_context *keep = nullptr;
     if (st->ctx) {
         (void)hipSetDevice(st->ctx->device);
         (void)ctx_resolve(st->ctx);          // the journal may name this state
         // the whole device, as hipFree waits: the caller's own streams may
         // still read the pointer of lmh_state_device_ptr, and the buffers are
         // used again without a hipFree in between
-        (void)hipDeviceSynchronize();
+        // (a wait that failed, e.g. beside a capture: nothing is kept)
+        if (hipDeviceSynchronize() == hipSuccess) keep = st->ctx;
         st->ctx->states.erase(st);
         if (st->ctx->tape.st == st) tape_clear(st->ctx);
     }
-    for (int q = 0; q < 3; ++q) sfree(st->ctx, st->buf[q], (size_t)st->ld * st->n);
-    sfree(st->ctx, st->pend_stval, (size_t)st->pend_cap_stval);
-    sfree(st->ctx, st->pend_sdiag, (size_t)st->pend_cap_sdiag);
-    sfree(st->ctx, st->pend_coef, 1);
+    for (int q = 0; q < 3; ++q) sfree(keep, st->buf[q], (size_t)st->ld * st->n);
+    sfree(keep, st->pend_stval, (size_t)st->pend_cap_stval);
+    sfree(keep, st->pend_sdiag, (size_t)st->pend_cap_sdiag);
+    sfree(keep, st->pend_coef, 1);
     delete st;
     return LMH_OK;
 }
