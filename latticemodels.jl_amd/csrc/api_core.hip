@@ -56,8 +56,7 @@ size_t spare_free_if(F match) {
         }
         (void)hipFree(v[k].p);          // waits for the device
         freed += v[k].bytes;
-        v[k] = v.back();
-        v.pop_back();
+        v.erase(v.begin() + k);
     }
     return freed;
 }
@@ -81,29 +80,35 @@ hipError_t spare_take(lmh_context *ctx, size_t bytes, void **out) {
         for (size_t k = 0; k < v.size(); ++k)
             if (v[k].ctx == ctx && v[k].bytes == bytes) {
                 *out = v[k].p;
-                v[k] = v.back();
-                v.pop_back();
+                v.erase(v.begin() + k);
                 return hipSuccess;
             }
     }
     return device_malloc(out, bytes);
 }
 
+// (the list is in the order in which buffers came: the first are the oldest)
 void spare_give(lmh_context *ctx, void *p, size_t bytes) {
-    if (ctx) {
+    if (ctx && bytes <= ctx->mem_total / 4) {
         std::lock_guard<std::mutex> lock(spare_mutex());
         auto &v = spares();
-        size_t mine = 0, held = 0;
-        for (const Spare &s : v) {
-            if (s.ctx == ctx) ++mine;
-            if (s.device == ctx->device) held += s.bytes;
-        }
-        if (mine < kSparesPerContext && held + bytes <= ctx->mem_total / 4) {
-            try {
-                v.push_back({ctx, ctx->device, p, bytes});
-                return;
-            } catch (const std::bad_alloc &) {
+        for (;;) {
+            size_t mine = 0, held = 0, first_mine = 0, first_here = v.size();
+            for (size_t k = v.size(); k-- > 0;) {
+                if (v[k].ctx == ctx) ++mine, first_mine = k;
+                if (v[k].device == ctx->device) held += v[k].bytes, first_here = k;
             }
+            const size_t out = mine >= kSparesPerContext              ? first_mine
+                               : held + bytes > ctx->mem_total / 4 ? first_here
+                                                                      : v.size();
+            if (out == v.size()) break;
+            (void)hipFree(v[out].p);
+            v.erase(v.begin() + out);
+        }
+        try {
+            v.push_back({ctx, ctx->device, p, bytes});
+            return;
+        } catch (const std::bad_alloc &) {
         }
     }
     (void)hipFree(p);

@@ -39,10 +39,6 @@ int hipfail(hipError_t e, const char *what);
 
 namespace lmhapi {
 
-// hipMalloc; when the device is full, the spare buffers on it (below) are
-// given back and the allocation is tried once more
-hipError_t device_malloc(void **p, size_t bytes);
-
 template <class T>
 hipError_t dalloc(T **p, size_t count) {
     *p = nullptr;
@@ -82,9 +78,10 @@ namespace lmhapi {
 // three N x N hipMalloc and hipFree (1.0 ms at N = 10^4, and at N = 28800,
 // once the driver has to clear the memory it hands out, 0.8 s).  Reuse stays
 // within one context, hence in its stream's order.  Bounded: kSparesPerContext
-// buffers of a context, a quarter of the device's memory over all contexts;
-// given back when the context's geometry changes or it is destroyed, when an
-// allocation fails, and before library calls that allocate by themselves.
+// buffers of a context, a quarter of the device's memory over all contexts,
+// the oldest making room for the newest; given back when the
+// context's geometry changes or it is destroyed, when an allocation fails
+// (device_malloc), and before library calls that allocate by themselves.
 constexpr size_t kSparesPerContext = 16;
 hipError_t spare_take(lmh_context *ctx, size_t bytes, void **out);
 void spare_give(lmh_context *ctx, void *p, size_t bytes);
