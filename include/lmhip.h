@@ -179,9 +179,14 @@ int lmh_solver_order(lmh_context *ctx, int32_t *K, double *s);
 int lmh_state_create(lmh_context *ctx, lmh_state **st);
 /* Waits for the device.  The state's buffers may stay with the context for
  * its next states and kets of that size (at most a quarter of the device's
- * memory over all contexts); they are freed when the context's geometry is
- * set again, when it is destroyed, and when the library needs the memory. */
+ * memory over all contexts, the oldest given up first); they are freed by
+ * lmh_release_spares, when the context's geometry is set again, when it is
+ * destroyed, and when the library needs the memory. */
 int lmh_state_destroy(lmh_state *st);
+/* Frees the buffers that destroyed states and kets left with the context
+ * (NULL: with every context), for other allocators in the process or other
+ * processes on the device. */
+int lmh_release_spares(lmh_context *ctx);
 /* Host <-> device copies of P (column-major, leading dimension ld >= N). */
 int lmh_state_upload(lmh_state *st, const double *P, int64_t ld);
 int lmh_state_download(lmh_state *st, double *P, int64_t ld);

@@ -382,6 +382,14 @@ int lmh_destroy(lmh_context *ctx) {
     return LMH_OK;
 }
 
+int lmh_release_spares(lmh_context *ctx) {
+    if (ctx)
+        spare_release_context(ctx);
+    else
+        spare_free_if([](const Spare &) { return true; });
+    return LMH_OK;
+}
+
 int lmh_set_progress(lmh_context *ctx, lmh_progress_fn fn, void *user) {
     int rc = check_ctx(ctx);
     if (rc) return rc;

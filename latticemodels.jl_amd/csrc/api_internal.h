@@ -79,8 +79,8 @@ namespace lmhapi {
 // once the driver has to clear the memory it hands out, 0.8 s).  Reuse stays
 // within one context, hence in its stream's order.  Bounded: kSparesPerContext
 // buffers of a context, a quarter of the device's memory over all contexts,
-// the oldest making room for the newest; given back when the
-// context's geometry changes or it is destroyed, when an allocation fails
+// the oldest making room for the newest; given back by lmh_release_spares, when
+// the context's geometry changes or it is destroyed, when an allocation fails
 // (device_malloc), and before library calls that allocate by themselves.
 constexpr size_t kSparesPerContext = 16;
 hipError_t spare_take(lmh_context *ctx, size_t bytes, void **out);

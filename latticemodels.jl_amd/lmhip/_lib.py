@@ -66,6 +66,7 @@ def lib():
         "lmh_solver_order": ([vp, ctypes.POINTER(i32), ctypes.POINTER(dbl)], ctypes.c_int),
         "lmh_state_create": ([vp, pvp], ctypes.c_int),
         "lmh_state_destroy": ([vp], ctypes.c_int),
+        "lmh_release_spares": ([vp], ctypes.c_int),
         "lmh_state_upload": ([vp, vp, i64], ctypes.c_int),
         "lmh_state_download": ([vp, vp, i64], ctypes.c_int),
         "lmh_state_copy": ([vp, vp], ctypes.c_int),

@@ -69,6 +69,12 @@ class Context:
         except Exception:
             pass
 
+    def release_spares(self):
+        """Gives the device memory back that destroyed states and kets left
+        here for the next ones (for torch or another process, say)."""
+        if self.h:
+            check(lib().lmh_release_spares(self.h))
+
     def set_hamiltonian(self, H):
         if isinstance(H, SparseHamiltonian):
             return self._set_sparse(H)

@@ -1,5 +1,5 @@
 """Buffers that destroyed states leave with their context: kept for the next
-state whatever smaller ones were left before."""
+state whatever smaller ones were left before, and given back on request."""
 import numpy as np
 import pytest
 import torch
@@ -40,3 +40,21 @@ def test_small_buffers_make_room_for_large_ones():
     assert abs(before - _free() - kept) <= 0.1 * STATE
     P.close()
     ctx.close()
+
+
+def test_spares_are_given_back_on_request():
+    H, n = _hamiltonian(), SIDE * SIDE
+    a, b = lmhip.Context(0), lmhip.Context(0)
+    for ctx in (a, b):
+        ctx.set_hamiltonian(H)
+    before = _free()
+    for ctx in (a, b):
+        lmhip.DensityMatrix(ctx, n).close()
+    assert before - _free() >= 1.9 * STATE
+    a.release_spares()
+    assert 0.9 * STATE <= before - _free() <= 1.1 * STATE
+    lmhip._lib.check(lmhip.lib().lmh_release_spares(None))
+    assert before - _free() <= 0.1 * STATE
+    # and the contexts go on
+    P = lmhip.DensityMatrix.from_array(a, np.eye(n, dtype=complex))
+    assert np.array_equal(P.to_numpy(), np.eye(n))
