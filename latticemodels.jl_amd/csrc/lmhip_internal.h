@@ -6,6 +6,8 @@
 #include <atomic>
 #include <cstdint>
 
+#include "strip_shape.h"
+
 namespace lmhapi {
 // hipMalloc; when the device is full, the spare buffers on it (api_internal.h)
 // are given back and the allocation is tried once more.  Every device
@@ -40,27 +42,6 @@ struct FieldComp {
     double a;     // B (Landau / symmetric) or flux (point fluxes)
     double px;
     double py;
-};
-
-// Grid-stencil geometry of H for the strip kernel (strip.hip): site
-// i = x * ly + y on an lx x ly grid, every stored entry of a row being the
-// diagonal or one of the four grid neighbours (y +- 1, x +- 1; across the
-// edges when px / py).  A strip is s consecutive sites of one x column
-// (y0 .. y0 + s - 1), a thread owns the strips of bx neighbouring x columns
-// (the last strip or block overlaps its neighbour when s does not divide ly,
-// or bx lx), a workgroup `cols` columns of P.
-struct StripGeom {
-    int lx = 0, ly = 0;
-    int lyp = 0;                // LDS length of bx x columns (bx * ly rounded up to odd)
-    int px = 0, py = 0;         // periodic along x / y
-    int s = 0;                  // sites per strip (0: H is not a grid stencil)
-    int bx = 0;                 // x columns per thread
-    int q = 0;                  // strips per x column
-    int nt = 0;                 // strips of a column of P = lx * q (strip k of x column x: k * lx + x)
-    int nthr = 0;               // threads per column of P
-    int threads = 0;            // workgroup size
-    int cols = 0;               // columns of P per workgroup
-    int region = 0;             // LDS entries per column (the last holds 0)
 };
 
 // Geometry + Hamiltonian in ELL layout on the device.

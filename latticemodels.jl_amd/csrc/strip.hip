@@ -56,23 +56,8 @@ namespace lmh {
 
 namespace {
 
-constexpr int kStripThreads = 512;      // 8 waves of 256 VGPRs per CU: one workgroup of 512, ..., eight of 64
-constexpr int kStripLdsBytes = 163840;
 constexpr int kStripMaxN = 10240;
-// blocks of x columns by sites: B(bx, s)
-#define LMH_STRIP_SHAPES(B) B(1, 20) B(2, 10) B(2, 8) B(2, 6) B(2, 4) B(4, 4)
-struct StripShape {
-    int bx, s;
-};
-constexpr StripShape kStripShapes[] = {
-#define LMH_STRIP_SHAPE(BX, S) {BX, S},
-    LMH_STRIP_SHAPES(LMH_STRIP_SHAPE)
-#undef LMH_STRIP_SHAPE
-};
 constexpr int strip_shape_id(int bx, int s) { return bx * 32 + s; }
-// a block with inner sites does not publish them: its neighbours must not
-// read them, so blocks may not overlap nor end early
-constexpr bool strip_whole(int bx, int s) { return bx > 2 && s > 2; }
 // (kStripMaxK: Horner coefficients passed with the launch or read from a
 // TaylorOut, lmhip_internal.h)
 
@@ -700,52 +685,6 @@ bool has_entry(const int32_t *col, int64_t n, int zmax, int64_t i, int64_t j) {
     for (int u = 0; u < zmax; ++u)
         if (col[(int64_t)u * n + i] == j) return true;
     return false;
-}
-
-// The block shape, workgroup size and columns per workgroup of an lx x ly
-// grid: those of least cost, the rounds of workgroups a CU takes (256 CUs of
-// 8 waves) times 25 (the barriers, latencies and launch of a round) plus its
-// waves' sites per thread (a wave takes its SIMD's time whether or not the
-// others have one), times 1.5 for whole strips (42 LDS reads per 20 sites
-// instead of 24), 1.05 for 4 x 4 (a few spills) and 0.97 for 2 x 10 (it fills a
-// batch's workgroups best).  Fitted to a step's launch (K = 8 twice): at
-// 64 x 64 2 x 8 482 us, 4 x 4 515, 2 x 4 550, 2 x 6 592; at 80 x 80 4 x 4 1094,
-// 2 x 8 1114, 2 x 10 1207; at 100 x 100 2 x 10 2252, 1 x 20 2715; at 37 x 23 2 x 4 30,
-// 2 x 8 36, 2 x 6 38; at 24 x 24 2 x 4 24, 2 x 8 30, 2 x 10 35.
-bool strip_shape(int64_t lx, int64_t ly, StripGeom *g) {
-    const int64_t n = lx * ly;
-    double best = 1e300;
-    for (const StripShape &sh : kStripShapes) {
-        if (sh.bx > lx || sh.s > ly) continue;
-        if (strip_whole(sh.bx, sh.s) && (lx % sh.bx || ly % sh.s)) continue;
-        const int64_t nbx = (lx + sh.bx - 1) / sh.bx, q = (ly + sh.s - 1) / sh.s, nthr = nbx * q;
-        const int64_t lyp = (sh.bx * ly) | 1, region = nbx * lyp + 1;
-        for (int64_t threads = (nthr + 63) / 64 * 64; threads <= kStripThreads; threads += 64) {
-            const int64_t cols = std::min<int64_t>(threads / nthr, kStripLdsBytes / (16 * region));
-            if (cols < 1) continue;
-            const int64_t groups = (n + cols - 1) / cols;
-            const int64_t fit = std::min<int64_t>(kStripThreads / threads, kStripLdsBytes / (16 * region * cols));
-            const int64_t per_cu = std::min<int64_t>(fit, (groups + 255) / 256);
-            const int64_t rounds = (groups + 256 * per_cu - 1) / (256 * per_cu);
-            const int64_t waves = (per_cu * (threads / 64) + 3) / 4 * 4;
-            const double cost = (double)rounds * (25.0 + (double)(waves * sh.bx * sh.s)) *
-                                (sh.bx == 1 ? 1.5 : (strip_whole(sh.bx, sh.s) ? 1.05 : (sh.s == 10 ? 0.97 : 1.0)));
-            if (cost >= best) continue;
-            best = cost;
-            g->lx = (int)lx;
-            g->ly = (int)ly;
-            g->lyp = (int)lyp;
-            g->bx = sh.bx;
-            g->s = sh.s;
-            g->q = (int)q;
-            g->nt = (int)(lx * q);
-            g->nthr = (int)nthr;
-            g->threads = (int)threads;
-            g->cols = (int)cols;
-            g->region = (int)region;
-        }
-    }
-    return best < 1e300;
 }
 
 }  // namespace
