@@ -85,6 +85,58 @@ hipError_t batch_strip_tables(lmh_batch *b) {
     return e;
 }
 
+// A member's H in the blocks that suit a batch (strip_batch_shape): its strips'
+// values are kept by block shape, so they are formed anew, and stay so until
+// the context's geometry is set again.  Steps outside the batch run on these blocks too,
+// at most a little slower.  Where some strip of the new shape is not uniform, or
+// the device is full, the member keeps the shape it has.
+int batch_blocks(lmh_context *cx) {
+    lmh::DevHam &h = cx->h;
+    lmh::StripGeom g = h.sg;
+    if (!lmh::strip_batch_shape(h.sg.lx, h.sg.ly, &g) || (g.bx == h.sg.bx && g.s == h.sg.s)) return LMH_OK;
+    // deferred passes hold strip values of the present shape
+    int rc = ctx_settle_all(cx);
+    if (rc) return rc;
+    HIP_TRY(hipStreamSynchronize(cx->stream), "member sync");
+    double2 *stval = nullptr;
+    double *sdiag = nullptr;
+    hipError_t e = dalloc(&stval, (size_t)4 * g.nt);
+    if (e == hipSuccess) e = dalloc(&sdiag, (size_t)g.s * g.nt);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        dfree(stval);
+        dfree(sdiag);
+        return LMH_OK;
+    }
+    const lmh::StripGeom old = h.sg;
+    h.sg = g;
+    std::swap(h.stval, stval);
+    std::swap(h.sdiag, sdiag);
+    auto form = [&](bool *uniform, bool *xreal) {
+        unsigned long long red[4] = {};
+        hipError_t er = lmh::launch_build_h(h, cx->stream);
+        if (er == hipSuccess) er = hipMemcpyAsync(red, h.red, sizeof red, hipMemcpyDeviceToHost, cx->stream);
+        const hipError_t es = hipStreamSynchronize(cx->stream);
+        *uniform = (red[3] & 1) == 0;
+        *xreal = (red[3] & 2) == 0;
+        return er == hipSuccess ? es : er;
+    };
+    bool uniform = false, xreal = false;
+    e = form(&uniform, &xreal);
+    if (e != hipSuccess || !uniform) {
+        h.sg = old;
+        std::swap(h.stval, stval);
+        std::swap(h.sdiag, sdiag);
+        if (e == hipSuccess) e = form(&uniform, &xreal);
+    }
+    dfree(stval);
+    dfree(sdiag);
+    if (e != hipSuccess) return hipfail(e, "batch strip values");
+    h.strip_xreal = xreal;
+    cx->solver_serial++;            // (another batch of this context refills its tables)
+    return LMH_OK;
+}
+
 // A member's H, K, s or dt changed since the tables were made (a time-
 // dependent H: the reference evaluates h(t) at every step of every
 // realisation, src/evolution.jl:238-250).  The kernel chosen for it at
@@ -177,9 +229,24 @@ int lmh_batch_create(lmh_batch **out, int64_t nmembers, lmh_context *const *ctxs
     std::map<int, std::vector<int>> byclass;
     b->member_kernel.assign(nmembers, -1);
     const bool use_strip = ctxs[0]->batch_strip != 0;
+    // a batch of fewer workgroups than the 256 CUs is over with its slowest one:
+    // the solo shapes' smaller blocks (64 members of 10 x 10: 38 us, 45 reshaped)
+    int64_t units = 0;
+    for (int64_t r = 0; r < nmembers; ++r) {
+        lmh::StripGeom g = ctxs[r]->h.sg;
+        if (ctxs[r]->h.strip_ok && g.s > 0 && lmh::strip_batch_shape(g.lx, g.ly, &g))
+            units += (ctxs[r]->h.n + lmh::strip_batch_cols(g) - 1) / lmh::strip_batch_cols(g);
+    }
+    const bool reshape = use_strip && units >= 256;
     for (int64_t r = 0; r < nmembers; ++r) {
         const lmh::DevHam &hr = ctxs[r]->h;
         if (use_strip && hr.strip_ok && hr.sg.s > 0) {
+            const int rc = reshape ? batch_blocks(ctxs[r]) : LMH_OK;
+            if (rc) {
+                batch_free(b);
+                delete b;
+                return rc;
+            }
             b->strip_members.push_back((int)r);
             b->member_kernel[r] = lmh::fused_strip_variant();
             continue;
@@ -188,6 +255,7 @@ int lmh_batch_create(lmh_batch **out, int64_t nmembers, lmh_context *const *ctxs
         const bool dict = dv >= 0 && hr.ndict > 0 && hr.dict_ok && lmh::fused_dict_fits(dv, hr.n, hr.ndict);
         byclass[dict ? dv : v].push_back((int)r);
     }
+    for (int64_t r = 0; r < nmembers; ++r) b->serials[r] = ctxs[r]->solver_serial;
     for (auto it = byclass.begin(); it != byclass.end();) {
         if (!lmh::fused_variant_is_dict(it->first)) {
             ++it;

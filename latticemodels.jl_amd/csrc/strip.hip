@@ -840,7 +840,7 @@ hipError_t strip_batch_table(const StripMemberDesc *m, int nm, void **d_args, in
         if (h.sg.s == 0 || h.n != (int64_t)h.sg.lx * h.sg.ly) return hipErrorInvalidValue;
         args[i] = strip_args(h, m[i].X, m[i].Y, m[i].ld, h.n, m[i].dts, m[i].K, m[i].reps);
         StripGeom &g = args[i].g;
-        g.cols = std::min(kStripThreads / g.nthr, (int)(kStripLdsBytes / ((size_t)g.region * sizeof(double2))));
+        g.cols = strip_batch_cols(g);
         need = std::max(need, (size_t)g.cols * g.region * sizeof(double2));
         ustart[i + 1] = ustart[i] + (h.n + g.cols - 1) / g.cols;
     }

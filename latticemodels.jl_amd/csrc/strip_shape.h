@@ -142,4 +142,37 @@ inline bool strip_shape(int64_t lx, int64_t ly, StripGeom *g) {
     return best < 1e300;
 }
 
+// columns of P in a batch's workgroup of 512 threads
+inline int strip_batch_cols(const StripGeom &g) {
+    return std::min(kStripThreads / g.nthr, (int)(kStripLdsBytes / (16 * (int64_t)g.region)));
+}
+
+// The block shape of a grid's members in a batch, where every workgroup has 512
+// threads and every term runs in one phase: the least cost per column of P of
+// an otherwise idle CU, fitted to uniform batches of seven shapes on 72 grids
+// (0.5 % behind the best in the mean).  The solo shape was up to twice as slow
+// there (us per step, N x members ~ 30000: 35 x 35 2 x 5 979, 2 x 8 1145;
+// 25 x 100 1 x 20 1920, 2 x 6 2095; 2 x 300 2 x 6 468, 2 x 4 634; 2 x 1000
+// 2 x 10 1395, 2 x 8 2756; 64 x 40 4 x 4 1777, 2 x 10 2144).
+inline bool strip_batch_shape(int64_t lx, int64_t ly, StripGeom *g) {
+    const int64_t n = lx * ly;
+    double best = 1e300;
+    StripGeom t = *g;
+    for (const StripShape &sh : kStripShapes) {
+        if (!strip_blocks(lx, ly, sh, &t) || !strip_shape_fits(t)) continue;
+        const int64_t cols = strip_batch_cols(t);
+        if (cols < 1) continue;
+        const int sites = t.bx * t.s;
+        const int64_t waves = ((t.nthr * cols + 63) / 64 + 3) / 4 * 4;
+        const double f = (t.bx == 4 ? 1.13 : sites == 16 ? 1.30 : sites == 20 ? 1.33 : 1.0) * (t.bx == 1 ? 1.11 : 1.0) *
+                         (1.0 + std::max(0.0, strip_conflict(t) - 2.0) * (t.s == 8 ? 0.39 : 0.23));
+        const double cost = (64.0 + 0.028 * (double)(n * cols) + (double)(waves * sites) * f) * (double)((n + cols - 1) / cols);
+        if (cost >= best) continue;
+        best = cost;
+        *g = t;
+    }
+    if (best < 1e300) strip_cost(g);        // (the workgroups of its launches outside the batch)
+    return best < 1e300;
+}
+
 }  // namespace lmh

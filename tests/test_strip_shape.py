@@ -23,16 +23,24 @@ int main() {
     while (std::scanf("%d %d", &lx, &ly) == 2) {
         StripGeom g;
         const bool ok = strip_shape(lx, ly, &g);
-        std::printf("%d %d %d %d %d %d %d\n", lx, ly, ok ? g.bx : 0, ok ? g.s : 0, g.threads, g.cols, g.nthr);
+        StripGeom b;
+        const bool okb = strip_batch_shape(lx, ly, &b);
+        std::printf("%d %d %d %d %d %d %d %d %d\n", lx, ly, ok ? g.bx : 0, ok ? g.s : 0, g.threads, g.cols, g.nthr,
+                    okb ? b.bx : 0, okb ? b.s : 0);
     }
     // every grid: what the kernel and its launcher take for granted
     long bad = 0, grids = 0, strips = 0;
     for (int x = 2; x <= 2560; ++x)
-        for (int y = 4; x * y <= 10240; ++y) {
+        for (int y = 4; x * y <= 10240; ++y)
+            for (int batch = 0; batch < 2; ++batch) {
             StripGeom g;
             ++grids;
-            if (!strip_shape(x, y, &g)) continue;
+            if (!(batch ? strip_batch_shape(x, y, &g) : strip_shape(x, y, &g))) continue;
             ++strips;
+            if (batch) {
+                const int c = strip_batch_cols(g);
+                if (c < 1 || c * g.nthr > 512 || 16L * g.region * c > 163840) ++bad;
+            }
             const int nbx = (x + g.bx - 1) / g.bx;
             const bool whole = x % g.bx == 0 && y % g.s == 0;
             if (g.lx != x || g.ly != y || g.bx > x || g.s > y || g.q != (y + g.s - 1) / g.s || g.nt != x * g.q ||
@@ -76,11 +84,27 @@ MEASURED = {
 }
 
 
+# the same in uniform batches (us per step of all members)
+BATCHES = {
+    (35, 35): {(2, 5): 979, (2, 6): 1066, (2, 4): 1071, (1, 20): 1116, (2, 8): 1145, (2, 10): 1162},
+    (64, 40): {(4, 4): 1777, (2, 5): 1854, (2, 8): 1925, (2, 6): 1990, (2, 10): 2144, (1, 20): 2187, (2, 4): 2631},
+    (25, 100): {(1, 20): 1920, (2, 8): 2072, (2, 6): 2095, (2, 10): 2265, (2, 4): 2833, (2, 5): 3165},
+    (5, 400): {(1, 20): 1566, (2, 10): 1801, (2, 5): 1835, (2, 6): 2035, (2, 8): 2495, (2, 4): 2969},
+    (2, 300): {(2, 6): 468, (2, 5): 471, (1, 20): 477, (2, 10): 490, (2, 4): 634, (2, 8): 858},
+    (2, 1000): {(2, 10): 1395, (1, 20): 1400, (2, 6): 1423, (2, 5): 1543, (2, 4): 1860, (2, 8): 2756},
+    (3, 340): {(1, 20): 869, (2, 10): 983, (2, 6): 986, (2, 5): 1124, (2, 4): 1181, (2, 8): 1397},
+}
+
+
 def test_every_grid_fits_and_measured_grids_take_a_fast_shape(tmp_path):
     rows, everything = _harness(tmp_path, list(MEASURED))
     assert everything.split()[3] == "0" and int(everything.split()[2]) > 30000
     for lx, ly, bx, s, *_ in rows:
         times = MEASURED[(lx, ly)]
+        assert times[(bx, s)] <= 1.1 * min(times.values()), (lx, ly, bx, s)
+    rows, _ = _harness(tmp_path, list(BATCHES))
+    for lx, ly, *_, bx, s in rows:
+        times = BATCHES[(lx, ly)]
         assert times[(bx, s)] <= 1.1 * min(times.values()), (lx, ly, bx, s)
 
 
