@@ -87,9 +87,9 @@ hipError_t batch_strip_tables(lmh_batch *b) {
 
 // A member's H in the blocks that suit a batch (strip_batch_shape): its strips'
 // values are kept by block shape, so they are formed anew, and stay so until
-// the context's geometry is set again.  Steps outside the batch run on these blocks too,
-// at most a little slower.  Where some strip of the new shape is not uniform, or
-// the device is full, the member keeps the shape it has.
+// the context's geometry is set again; its steps outside the batch run on these
+// blocks too.  Where some strip of the new shape is not uniform, or the device
+// is full, the member keeps the shape it has.
 int batch_blocks(lmh_context *cx) {
     lmh::DevHam &h = cx->h;
     lmh::StripGeom g = h.sg;

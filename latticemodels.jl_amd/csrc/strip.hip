@@ -36,9 +36,10 @@
 // The workgroup is persistent over its share of the columns.
 //
 // Whether H qualifies is decided twice: the pattern on the host when the
-// geometry is set (strip_detect), and the values after every H build on the
-// device (h_check_kernel: every used bond of a strip's direction equal
-// to the strip's value, bit for bit).  When either fails, the fused passes
+// geometry is set (strip_detect, which also picks the block shape:
+// strip_shape.h), and the values after every H build on the device
+// (h_check_kernel: every used bond of a strip's direction equal to the strip's
+// value, and that the conjugate of its partner's, bit for bit).  When either fails, the fused passes
 // run the general kernels of fused.hip, so this kernel changes speed, never
 // results.  Reference step: src/evolution.jl:73-78 (U P U' with U from
 // myexp!, :93-128); the polynomial is the reference's order-K Taylor
@@ -765,13 +766,15 @@ hipError_t launch_args(const DevHam &h, StripArgs &a, int64_t ncols, bool tout, 
     const int64_t per_cu = std::min<int64_t>(kStripThreads / g.threads, kStripLdsBytes / (int64_t)lds);
     const int64_t np = std::min<int64_t>(groups, per_cu * std::max(cus, 1));
     a.nprog = ((np + kNumXCD - 1) / kNumXCD) * kNumXCD;
-    // half a column period in shader cycles (measured at N = 10^4, S = 20:
-    // ~310 cycles per site and term, ~3.3 cycles per site for the load and
-    // store), when each workgroup has several column groups to do
+    // half a column period in shader cycles (at N = 10^4 in 2 x 10 blocks: 220
+    // cycles per site of a block and term, 6 per site of a column for its load
+    // and store), when each workgroup has several column groups to do (a step
+    // at 100 x 100: 2410 us without, 2370 with it, 2450 with twice as much; at
+    // 96 x 96 and below within 1 % of none)
     int64_t terms = 0;
     for (int q = 0; q < a.npoly; ++q) terms += (int64_t)a.poly[q].K * a.poly[q].reps;
     a.stagger = per_cu == 1 && groups >= 4 * a.nprog
-                    ? (int64_t)((310.0 * terms * g.bx * g.s + 3.3 * (double)h.n * g.cols) / 2.0)
+                    ? (int64_t)((220.0 * terms * g.bx * g.s + 6.0 * (double)h.n * g.cols) / 2.0)
                     : 0;
     return dispatch_s(tout, a.xreal != 0, a, lds, st);
 }
