@@ -179,7 +179,8 @@ int lmh_solver_order(lmh_context *ctx, int32_t *K, double *s);
 int lmh_state_create(lmh_context *ctx, lmh_state **st);
 /* Waits for the device.  The state's buffers may stay with the context for
  * its next states and kets of that size (at most a quarter of the device's
- * memory over all contexts, the oldest given up first); they are freed by
+ * memory over all contexts, the context's oldest of other sizes given up
+ * first); they are freed by
  * lmh_release_spares, when the context's geometry is set again, when it is
  * destroyed, and when the library needs the memory. */
 int lmh_state_destroy(lmh_state *st);

@@ -89,26 +89,29 @@ hipError_t spare_take(lmh_context *ctx, size_t bytes, void **out) {
 
 // (the list is in the order in which buffers came: the first are the oldest)
 void spare_give(lmh_context *ctx, void *p, size_t bytes) {
-    if (ctx && bytes <= ctx->mem_total / 4) {
+    if (ctx) {
         std::lock_guard<std::mutex> lock(spare_mutex());
         auto &v = spares();
         for (;;) {
-            size_t mine = 0, held = 0, first_mine = 0, first_here = v.size();
+            size_t mine = 0, held = 0, other = v.size();     // other: the context's oldest of another size
             for (size_t k = v.size(); k-- > 0;) {
-                if (v[k].ctx == ctx) ++mine, first_mine = k;
-                if (v[k].device == ctx->device) held += v[k].bytes, first_here = k;
+                if (v[k].ctx == ctx) {
+                    ++mine;
+                    if (v[k].bytes != bytes) other = k;
+                }
+                if (v[k].device == ctx->device) held += v[k].bytes;
             }
-            const size_t out = mine >= kSparesPerContext              ? first_mine
-                               : held + bytes > ctx->mem_total / 4 ? first_here
-                                                                      : v.size();
-            if (out == v.size()) break;
-            (void)hipFree(v[out].p);
-            v.erase(v.begin() + out);
-        }
-        try {
-            v.push_back({ctx, ctx->device, p, bytes});
-            return;
-        } catch (const std::bad_alloc &) {
+            if (mine < kSparesPerContext && held + bytes <= ctx->mem_total / 4) {
+                try {
+                    v.push_back({ctx, ctx->device, p, bytes});
+                    return;
+                } catch (const std::bad_alloc &) {
+                    break;
+                }
+            }
+            if (other == v.size()) break;
+            (void)hipFree(v[other].p);
+            v.erase(v.begin() + other);
         }
     }
     (void)hipFree(p);

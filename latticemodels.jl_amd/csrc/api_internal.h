@@ -79,7 +79,9 @@ namespace lmhapi {
 // once the driver has to clear the memory it hands out, 0.8 s).  Reuse stays
 // within one context, hence in its stream's order.  Bounded: kSparesPerContext
 // buffers of a context, a quarter of the device's memory over all contexts,
-// the oldest making room for the newest; given back by lmh_release_spares, when
+// a context's oldest of other sizes making room for the newest (other
+// contexts' do not: two that take turns would free and allocate every time,
+// 1.1 s more a pass at N = 28800); given back by lmh_release_spares, when
 // the context's geometry changes or it is destroyed, when an allocation fails
 // (device_malloc), and before library calls that allocate by themselves.
 constexpr size_t kSparesPerContext = 16;
