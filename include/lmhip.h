@@ -178,11 +178,11 @@ int lmh_solver_order(lmh_context *ctx, int32_t *K, double *s);
  * src/evolution.jl:80,188-196).  Contents undefined until uploaded. */
 int lmh_state_create(lmh_context *ctx, lmh_state **st);
 /* Waits for the device.  The state's buffers may stay with the context for
- * its next states and kets of that size (at most a quarter of the device's
- * memory over all contexts, the context's oldest of other sizes given up
- * first); they are freed by
- * lmh_release_spares, when the context's geometry is set again, when it is
- * destroyed, and when the library needs the memory. */
+ * its next states and kets of that size (at most 16, and a quarter of the
+ * device's memory over all contexts; the context's oldest of other sizes are
+ * given up first).  They are freed by lmh_release_spares, when the context's
+ * geometry is set again, when it is destroyed, and when the library needs the
+ * memory. */
 int lmh_state_destroy(lmh_state *st);
 /* Frees the buffers that destroyed states and kets left with the context
  * (NULL: with every context), for other allocators in the process or other

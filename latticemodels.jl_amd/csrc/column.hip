@@ -416,8 +416,8 @@ bool column_variant_valid(int v, int64_t n, int zmax) {
 // 634, 2888 713 / 673, 3528 942 / 1373, 4232 1794 / 1823, 5000 2233 / 2184.
 // So from 6 slots on a sixth row of 512 threads goes to the general kernel
 // (which has 1024 with three each), except that with 9 a wave's worth of it
-// costs nothing; rows past the seventh with 7 or 8 slots, past the eighth with 5 or
-// 6 (with 9 the general kernel loads 12 slots and both are within 2 %).
+// costs nothing; rows past the seventh with 7 or 8 slots, past the eighth with
+// 5 or 6 (with 9 the general kernel loads 12 slots and both are within 2 %).
 // Few columns (at most two to a CU) are one round of either, and the streamed
 // rows the shorter one up to more of them (48 kets: 5 slots N = 3698 50 / 66;
 // 7 slots 3698 69 / 73; 8 slots 2704 55 / 59, 3600 74 / 74, 4096 80 / 75;

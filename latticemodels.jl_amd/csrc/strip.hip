@@ -39,9 +39,9 @@
 // geometry is set (strip_detect, which also picks the block shape:
 // strip_shape.h), and the values after every H build on the device
 // (h_check_kernel: every used bond of a strip's direction equal to the strip's
-// value, and that the conjugate of its partner's, bit for bit).  When either fails, the fused passes
-// run the general kernels of fused.hip, so this kernel changes speed, never
-// results.  Reference step: src/evolution.jl:73-78 (U P U' with U from
+// value, and that the conjugate of its partner's, bit for bit).  When either
+// fails, the fused passes run the kernels of column.hip or fused.hip, so this
+// kernel changes speed, never results.  Reference step: src/evolution.jl:73-78 (U P U' with U from
 // myexp!, :93-128); the polynomial is the reference's order-K Taylor
 // polynomial evaluated in Horner form.
 #include <algorithm>
